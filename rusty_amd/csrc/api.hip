@@ -451,7 +451,7 @@ static int matmul_common(rq_ctx *ctx, int variant, const float *a, const float *
     if (!mul_ok(m, k, &t) || !mul_ok(k, n, &t) || !mul_ok(m, n, &t)) return fail(RQ_ERR_SHAPE, "shape overflows");
     if (m == 0 || n == 0) return RQ_OK;
     if (!out || (k > 0 && (!a || !b))) return fail(RQ_ERR_INVALID_ARGUMENT, "null pointer");
-    return launch_matmul_f32(variant, a, b, out, m, k, n, pick(ctx, stream));
+    return launch_matmul_f32(variant, a, b, out, m, k, n, ctx->num_cus, pick(ctx, stream));
 }
 
 int rq_matmul(rq_ctx *ctx, const float *a, const float *b, float *out, int64_t m, int64_t k, int64_t n,

@@ -315,7 +315,7 @@ int lora_run(rq_ctx *ctx, const rq_qweight *w, const void *x, rq_dtype x_dtype, 
         // t = x . A [m, rank]: one fma chain per output, k ascending.  fp16 x:
         // the chain kernel widens it while staging where it serves the shape,
         // else x is widened to f32 first (exact either way).
-        st = x_dtype == RQ_F16 ? launch_matmul_f32_ah(static_cast<const _Float16 *>(x), lora_a, tv, m, K, rank, s)
+        st = x_dtype == RQ_F16 ? launch_matmul_f32_ah(static_cast<const _Float16 *>(x), lora_a, tv, m, K, rank, ctx->num_cus, s)
                                : RQ_ERR_UNSUPPORTED;
         if (st == RQ_ERR_UNSUPPORTED) {
             const float *xf = static_cast<const float *>(x);
@@ -327,7 +327,7 @@ int lora_run(rq_ctx *ctx, const rq_qweight *w, const void *x, rq_dtype x_dtype, 
                 }
                 xf = w32;
             }
-            st = launch_matmul_f32(MM_AB, xf, lora_a, tv, m, K, rank, s);
+            st = launch_matmul_f32(MM_AB, xf, lora_a, tv, m, K, rank, ctx->num_cus, s);
         }
         if (st != RQ_OK) return st;
     }

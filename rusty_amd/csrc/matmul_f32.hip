@@ -7,13 +7,20 @@
 // Every output is one f32 accumulator updated in ascending k with a fused
 // multiply-add, the order all three WGSL kernels use, so results are
 // bit-identical to a sequential k-ascending fma loop regardless of tiling.
-// Tiles are 64x64 per 256-thread block with 4x4 outputs per thread (16x the
-// reuse of the reference's 16x16 one-output-per-invocation tiles); operands
-// are staged through LDS k-major so the inner loop reads broadcast rows.
-// Out-of-range rows/columns/k load as zero, which leaves every in-range
-// accumulator unchanged.
+// Most calls run on the f32 matrix cores (matmul_mfma.hpp), which keep that
+// arithmetic; the VALU kernels below serve what they are faster at (see
+// route()): the tiled one products of a few k-steps, the chains a few outputs
+// over a long k.
+//
+// The tiled kernel: 64x64 tiles per 256-thread block with 4x4 outputs per
+// thread; operands are staged through LDS k-major so the inner loop reads
+// broadcast rows.  Out-of-range rows/columns/k load as zero, which leaves
+// every in-range accumulator unchanged.
+#include <type_traits>
+
 #include "common.hpp"
 #include "lds_dma.hpp"
+#include "matmul_mfma.hpp"
 
 namespace rq {
 namespace {
@@ -127,11 +134,10 @@ __global__ __launch_bounds__(TH) void k_matmul_f32(const float *__restrict__ a, 
         }
 }
 
-// Grids of few 64x64 tiles (few rows or few columns: configs[0]'s 8 x 1024,
-// a LoRA adapter's x . A with 16 columns) leave most CUs idle while each
-// block walks all of k alone, 16 k-steps per pair of barriers.  There, a
+// One 16x16 tile of outputs over a long k (a LoRA adapter's x . A at decode)
+// is a single chain of dependent fmas whatever runs it: a
 // block owns a TR x TC output tile, one output per thread (TR * TC = 256),
-// and the same k-ascending fma chain per output runs over k-chunks of KC
+// and the k-ascending fma chain per output runs over k-chunks of KC
 // staged in LDS by all the block's threads (coalesced along the operand's
 // contiguous dimension); the next chunk's loads are in registers before the
 // current chunk's chains run.  A is staged [TR][KC + 4] and B transposed,
@@ -153,7 +159,7 @@ __device__ __forceinline__ float bload(__amdgpu_buffer_rsrc_t r, uint32_t voff, 
 }
 
 template <int TC>
-constexpr int chain_kc() { return TC == 16 || TC == 32 ? 512 : 256; }  // 64-80 KiB of LDS per chunk
+constexpr int chain_kc() { return TC == 16 ? 512 : 256; }  // 40-64 KiB of LDS per chunk
 
 // AH: A holds fp16 values (MM_AB only), loaded as 2-byte elements and
 // widened exactly when staged -- the f32 matmul of the widened copy, without
@@ -290,42 +296,36 @@ __global__ __launch_bounds__(TH) void k_matmul_f32_chain(const void *__restrict_
     if (r < m && c < n) out[r * n + c] = acc;
 }
 
-// The same chains fed through an LDS ring of NS chunks of KC = 256 k-steps
-// filled by global -> LDS DMA (16 bytes per lane, no registers held), so
-// NS - 1 chunks are in flight while one is multiplied.  A chain advances one
-// dependent fma per 8.4 cycles (MI355X, one wave), 0.9 us per chunk, while a
-// chunk's loads take about two: with one chunk in flight (the register-
-// staged kernel above) every chunk waited for its data.  Each operand keeps
-// its stored layout in LDS, as the DMA writes lane pieces contiguously:
-//  * rows along k (A of MM_AB and MM_ABT, B of MM_ABT): [R][KC + 4], each
-//    row's chunk one 1 KiB DMA unit; the chain reads four k-steps per ds_read_b128;
-//  * rows along the outputs (A of MM_ATB, B of MM_AB and MM_ATB): [KC][C],
-//    C = TR or TC columns, a unit covering 256 / C k-rows; the chain reads
-//    one k-step per element (paired into ds_read2_b32).
+// The same chains for C = A.B^T fed through an LDS ring of NS chunks of KC =
+// 256 k-steps filled by global -> LDS DMA (16 bytes per lane, no registers
+// held), so NS - 1 chunks are in flight while one is multiplied.  A chain
+// advances one dependent fma per 8.4 cycles (MI355X, one wave), 0.9 us per
+// chunk, while a chunk's loads take about two: with one chunk in flight (the
+// register-staged kernel above) every chunk waited for its data.  Both
+// operands keep their rows along k in LDS, as the DMA writes lane pieces
+// contiguously: [R][KC + 4], each row's chunk one 1 KiB DMA unit; the chain
+// reads four k-steps per ds_read_b128.
 // Units of a chunk: TR for A, TC for B, wave w issuing units w, w + 4, ...
-// Positions past an operand read as zero or land in rows, columns or k that
-// no stored output uses (as above); the dummy DMAs of chunks past K use an
-// offset beyond every resource (operands < 2 GiB, chain_fits).  Requires
-// 16-byte aligned operands and row pitches (ring_ok).
+// Positions past an operand read as zero or land in rows or k that no stored
+// output uses (as above); the dummy DMAs of chunks past K use an offset
+// beyond every resource (operands < 2 GiB, chain_fits).  Requires 16-byte
+// aligned operands and row pitches (ring_ok).
 constexpr int RKC = 256;
 constexpr uint32_t kOOBf = 0x80000000u;  // past every operand resource (operands < 2 GiB)
-template <int V, int TC>
+template <int TC>
 struct RingShape {
     static constexpr int TR = TH / TC;
-    static constexpr bool AK = V != MM_ATB;  // A stored with rows along k
-    static constexpr bool BK = V == MM_ABT;  // B stored with rows along k
-    static constexpr int SA = AK ? TR * (RKC + 4) : RKC * TR;  // floats per stage
-    static constexpr int SB = BK ? TC * (RKC + 4) : RKC * TC;
+    static constexpr int SA = TR * (RKC + 4), SB = TC * (RKC + 4);  // floats per stage
     static constexpr int ST = SA + SB;
     static constexpr int NS = 4 * ST * 4 <= 140 * 1024 ? 4 : 3;
     static constexpr int OPS = (TR + TC) / 4;  // DMA units per wave per chunk
     static_assert(3 * ST * 4 <= 140 * 1024 && (TR + TC) % 4 == 0, "ring does not fit");
 };
 
-template <int V, int TC>
+template <int TC>
 __global__ __launch_bounds__(TH) void k_matmul_f32_ring(const float *__restrict__ a, const float *__restrict__ b,
                                                         float *__restrict__ out, int64_t m, int64_t k, int64_t n) {
-    using RS = RingShape<V, TC>;
+    using RS = RingShape<TC>;
     constexpr int TR = RS::TR, NS = RS::NS, OPS = RS::OPS, SA = RS::SA, ST = RS::ST, AS = RKC + 4;
     constexpr int G = 32;
     // (+ G: the chains' reads one register set past a chunk stay inside the ring)
@@ -334,20 +334,14 @@ __global__ __launch_bounds__(TH) void k_matmul_f32_ring(const float *__restrict_
     const int wave = __builtin_amdgcn_readfirstlane(t / 64);
     const int64_t r0 = (int64_t)blockIdx.y * TR, c0 = (int64_t)blockIdx.x * TC;
     const int tr = t / TC, tc = t % TC;
-    const uint32_t K = (uint32_t)k, M = (uint32_t)m, N = (uint32_t)n;
+    const uint32_t K = (uint32_t)k;
     const auto rsa = make_rsrc(a, (uint32_t)(m * k * 4)), rsb = make_rsrc(b, (uint32_t)(k * n * 4));
     const uint32_t ring0 = lds_addr(&ring[0]);
     const int nck = (int)((k + RKC - 1) / RKC);
 
-    // Byte offset of this lane's piece of unit i of chunk c (see above):
-    // rows along k: row i of the panel, k = c KC + 4 lane; rows along the
-    // outputs: k-row c KC + i (256 / C) + lane / (C / 4), columns 4 (lane % (C / 4)).
+    // Byte offset of this lane's piece of row i of a panel in chunk c: k = c KC + 4 lane.
     auto off_k = [&](uint32_t row0, uint32_t ld, int i, int c) {
         return (((row0 + (uint32_t)i) * ld + (uint32_t)(c * RKC)) + 4u * (uint32_t)lane) * 4u;
-    };
-    auto off_o = [&](uint32_t col0, uint32_t ld, int C, int i, int c) {
-        const uint32_t kr = (uint32_t)(c * RKC + i * (256 / C) + lane / (C / 4));
-        return (kr * ld + col0 + 4u * (uint32_t)(lane % (C / 4))) * 4u;
     };
     auto issue = [&](int c) {
         const int s = c % NS;
@@ -356,13 +350,13 @@ __global__ __launch_bounds__(TH) void k_matmul_f32_ring(const float *__restrict_
         for (int q = 0; q < OPS; ++q) {
             const int u = wave + 4 * q;  // wave-uniform
             if (u < TR) {
-                const uint32_t dst = ring0 + (uint32_t)(s * ST) * 4u + (RS::AK ? (uint32_t)(u * AS) * 4u : (uint32_t)u * 1024u);
-                const uint32_t off = RS::AK ? off_k((uint32_t)r0, K, u, c) : off_o((uint32_t)r0, M, TR, u, c);
+                const uint32_t dst = ring0 + (uint32_t)(s * ST) * 4u + (uint32_t)(u * AS) * 4u;
+                const uint32_t off = off_k((uint32_t)r0, K, u, c);
                 dma16(rsa, dst, live ? off : kOOBf);
             } else {
                 const int i = u - TR;
-                const uint32_t dst = ring0 + (uint32_t)(s * ST + SA) * 4u + (RS::BK ? (uint32_t)(i * AS) * 4u : (uint32_t)i * 1024u);
-                const uint32_t off = RS::BK ? off_k((uint32_t)c0, K, i, c) : off_o((uint32_t)c0, N, TC, i, c);
+                const uint32_t dst = ring0 + (uint32_t)(s * ST + SA) * 4u + (uint32_t)(i * AS) * 4u;
+                const uint32_t off = off_k((uint32_t)c0, K, i, c);
                 dma16(rsb, dst, live ? off : kOOBf);
             }
         }
@@ -378,34 +372,24 @@ __global__ __launch_bounds__(TH) void k_matmul_f32_ring(const float *__restrict_
         issue(c + NS - 1);             // into chunk c - 1's stage
         if (idle) continue;
         const float *sa = ring + (c % NS) * ST, *sb = sa + SA;
-        auto a_at = [&](int kk) -> const float * { return RS::AK ? sa + tr * AS + kk : sa + kk * TR + tr; };
-        auto b_at = [&](int kk) -> const float * { return RS::BK ? sb + tc * AS + kk : sb + kk * TC + tc; };
+        auto a_at = [&](int kk) -> const float * { return sa + tr * AS + kk; };
+        auto b_at = [&](int kk) -> const float * { return sb + tc * AS + kk; };
         const int64_t k0 = (int64_t)c * RKC;
         if (k0 + RKC <= k) {
             float xa0[G], xb0[G], xa1[G], xb1[G];
             auto rd = [&](float *xa, float *xb, int kk) {
 #pragma unroll
                 for (int i = 0; i < G; i += 4) {
-                    if constexpr (RS::AK) {
-                        const float4 v = *reinterpret_cast<const float4 *>(a_at(kk + i));
-                        xa[i] = v.x;
-                        xa[i + 1] = v.y;
-                        xa[i + 2] = v.z;
-                        xa[i + 3] = v.w;
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) xa[i + j] = *a_at(kk + i + j);
-                    }
-                    if constexpr (RS::BK) {
-                        const float4 u = *reinterpret_cast<const float4 *>(b_at(kk + i));
-                        xb[i] = u.x;
-                        xb[i + 1] = u.y;
-                        xb[i + 2] = u.z;
-                        xb[i + 3] = u.w;
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) xb[i + j] = *b_at(kk + i + j);
-                    }
+                    const float4 v = *reinterpret_cast<const float4 *>(a_at(kk + i));
+                    xa[i] = v.x;
+                    xa[i + 1] = v.y;
+                    xa[i + 2] = v.z;
+                    xa[i + 3] = v.w;
+                    const float4 u = *reinterpret_cast<const float4 *>(b_at(kk + i));
+                    xb[i] = u.x;
+                    xb[i + 1] = u.y;
+                    xb[i + 2] = u.z;
+                    xb[i + 3] = u.w;
                 }
             };
             auto fm = [&](const float *xa, const float *xb) {
@@ -438,22 +422,10 @@ bool chain_fits(int64_t m, int64_t k, int64_t n) {
     return (m + 64) * (k + 1024) < lim && (k + 1024) * (n + 128) < lim;
 }
 
-// The ring kernel's 16-byte DMA pieces: aligned operands, and every row
-// along which pieces are taken a multiple of 4 floats long.  At n <= 16 with
-// B stored along the outputs (one LDS read per k-step and element) the four
-// waves' reads outweigh the latency the ring hides, and the register-staged
-// kernel stays (MI355X, us, ring / register-staged: 512x4096x16 34.3 / 27.7;
-// 8x1024x1024 9.7 / 13.2, 1x4096x4096 26.0 / 45.6, 16x4096x4096 35.5 / 49;
-// C = A.B^T 512x4096x16 25.8 / 27.0).
-bool ring_ok(int v, const float *a, const float *b, int64_t m, int64_t k, int64_t n) {
-    if (!aligned(a, 16) || !aligned(b, 16)) return false;
-    if (v != MM_ABT && n <= 16) return false;
-    if (v == MM_ATB) return m % 4 == 0 && n % 4 == 0;
-    if (v == MM_ABT) return k % 4 == 0;
-    return k % 4 == 0 && n % 4 == 0;
-}
+// The ring kernel's 16-byte DMA pieces: aligned operands, rows a multiple of
+// 4 floats long.
+bool ring_ok(const float *a, const float *b, int64_t k) { return aligned(a, 16) && aligned(b, 16) && k % 4 == 0; }
 
-template <int V>
 int launch_ring(const float *a, const float *b, float *out, int64_t m, int64_t k, int64_t n, hipStream_t s) {
     const int tc = n > 16 ? 32 : (n > 8 ? 16 : 8);
     const int64_t gx = cdiv(n, tc), gy = cdiv(m, TH / tc);
@@ -461,9 +433,9 @@ int launch_ring(const float *a, const float *b, float *out, int64_t m, int64_t k
         return fail(RQ_ERR_SHAPE, "matmul grid too large (m=%lld n=%lld)", (long long)m, (long long)n);
     const dim3 grid((unsigned)gx, (unsigned)gy);
     switch (tc) {
-    case 32: hipLaunchKernelGGL((k_matmul_f32_ring<V, 32>), grid, dim3(TH), 0, s, a, b, out, m, k, n); break;
-    case 16: hipLaunchKernelGGL((k_matmul_f32_ring<V, 16>), grid, dim3(TH), 0, s, a, b, out, m, k, n); break;
-    default: hipLaunchKernelGGL((k_matmul_f32_ring<V, 8>), grid, dim3(TH), 0, s, a, b, out, m, k, n); break;
+    case 32: hipLaunchKernelGGL((k_matmul_f32_ring<32>), grid, dim3(TH), 0, s, a, b, out, m, k, n); break;
+    case 16: hipLaunchKernelGGL((k_matmul_f32_ring<16>), grid, dim3(TH), 0, s, a, b, out, m, k, n); break;
+    default: hipLaunchKernelGGL((k_matmul_f32_ring<8>), grid, dim3(TH), 0, s, a, b, out, m, k, n); break;
     }
     RQ_LAUNCH_CHECK();
     return RQ_OK;
@@ -471,41 +443,69 @@ int launch_ring(const float *a, const float *b, float *out, int64_t m, int64_t k
 
 template <int V, bool AH = false>
 int launch_chain(const void *a, const float *b, float *out, int64_t m, int64_t k, int64_t n, hipStream_t s) {
-    const int tc = n >= 64 ? 64 : (n > 16 ? 32 : (n > 8 ? 16 : 8));
+    const int tc = n > 8 ? 16 : 8;  // n <= 16 (route)
     const int64_t gx = cdiv(n, tc), gy = cdiv(m, TH / tc);
     if (gx > 0x7fffffff || gy > 65535)
         return fail(RQ_ERR_SHAPE, "matmul grid too large (m=%lld n=%lld)", (long long)m, (long long)n);
     const dim3 grid((unsigned)gx, (unsigned)gy);
-    switch (tc) {
-    case 64: hipLaunchKernelGGL((k_matmul_f32_chain<V, 64, AH>), grid, dim3(TH), 0, s, a, b, out, m, k, n); break;
-    case 32: hipLaunchKernelGGL((k_matmul_f32_chain<V, 32, AH>), grid, dim3(TH), 0, s, a, b, out, m, k, n); break;
-    case 16: hipLaunchKernelGGL((k_matmul_f32_chain<V, 16, AH>), grid, dim3(TH), 0, s, a, b, out, m, k, n); break;
-    default: hipLaunchKernelGGL((k_matmul_f32_chain<V, 8, AH>), grid, dim3(TH), 0, s, a, b, out, m, k, n); break;
-    }
+    if (tc == 16) hipLaunchKernelGGL((k_matmul_f32_chain<V, 16, AH>), grid, dim3(TH), 0, s, a, b, out, m, k, n);
+    else hipLaunchKernelGGL((k_matmul_f32_chain<V, 8, AH>), grid, dim3(TH), 0, s, a, b, out, m, k, n);
     RQ_LAUNCH_CHECK();
     return RQ_OK;
+}
+
+// Offsets within a panel stay below 2^29 elements (ChainSpan): rows of up to
+// 4 M elements along k, 8 M along the outputs.
+bool mfma_fits(int v, int64_t m, int64_t k, int64_t n) {
+    const int64_t lim = (int64_t)1 << 29;
+    return (v == MM_ATB ? m * 64 < lim : k * 128 < lim) && (v == MM_ABT ? k * 128 < lim : n * 64 < lim) &&
+           cdiv(m, 16) * cdiv(n, 16) < ((int64_t)1 << 31);
+}
+// Which kernel serves a product, measured on MI355X (us, VALU kernels ->
+// matrix cores, AB / ABT / ATB unless stated):
+//  * k <= 16, or k <= 48 with over 2^21 outputs: the tiled VALU kernel.  Such
+//    a product is its output's write, and the tiled kernel's small LDS keeps
+//    more blocks in flight (4096x16x4096 18.0 / 17.7 / 16.4 -> 33.3 / 34.1 /
+//    31.1, 4096x48x4096 33 -> 41; 512x32x4096 6.3 -> 5.8, 4096x64x4096 40.6 -> 39.5);
+//  * A . B^T with at most 65536 outputs and 16-byte pieces: the ring chains,
+//    which have more k in flight (8x1024x1024 7.3 -> 8.0, 1x4096x4096 19.4 ->
+//    24.8, 16x512x4096 5.0 -> 5.4; even at 16x4096x4096 25.4 -> 25.1);
+//  * over 256 k for a single 16x16 tile: the register-staged chains
+//    (1x4096x16 22.3 / 18.6 / 22.3 -> 24.4 / 24.2 / 42.2);
+//  * everything else: the matrix cores (4096^3 2270 / 2185 / 2223 -> 978 /
+//    998 / 966, 512x4096x4096 368 / 329 / 360 -> 146 / 146 / 139, 1024^3 74 /
+//    66 / 74 -> 21, 300x1000x777 72 / 64 / 72 -> 10.2 / 9.0 / 10.1,
+//    537x2773x2853 241 / 224 / 245 -> 93 / 87 / 101, 8x4096x11008 286 / 254 /
+//    292 -> 28, 512x4096x16 27.3 / 26.1 / 28.0 -> 24.7 / 24.7 / 27.0).
+enum Route { ROUTE_TILED, ROUTE_CHAIN, ROUTE_RING, ROUTE_MFMA };
+template <typename TA>
+Route route(int v, const TA *a, const float *b, int64_t m, int64_t k, int64_t n) {
+    if (k <= 16 || (k <= 48 && m * n > ((int64_t)1 << 21))) return ROUTE_TILED;
+    const bool chain = k > 64 && chain_fits(m, k, n);
+    if constexpr (std::is_same_v<TA, float>)
+        if (chain && v == MM_ABT && m * n <= 65536 && ring_ok(a, b, k)) return ROUTE_RING;
+    const int64_t tiles = cdiv(m, 16) * cdiv(n, 16);
+    if (chain && k > 256 && tiles <= 1)
+        return ROUTE_CHAIN;
+    return mfma_fits(v, m, k, n) ? ROUTE_MFMA : ROUTE_TILED;
 }
 
 }  // namespace
 
 int launch_matmul_f32(int variant, const float *a, const float *b, float *out, int64_t m, int64_t k, int64_t n,
-                      hipStream_t s) {
+                      int num_cus, hipStream_t s) {
     if (m == 0 || n == 0) return RQ_OK;
-    const int64_t gx = cdiv(n, BN), gy = cdiv(m, BM);
-    // The chain kernels for few outputs or few tiles with more than a few
-    // k-steps, measured (MI355X, us, chain / tiled, C = A.B): 8x1024x1024
-    // 9.7 / 86, 1x4096x16 22.5 / 335, 16x4096x4096 35.5 / 342, 64x1024x1024
-    // 9.9 / 86; with more outputs the tiled kernel's reuse wins (256x1024x4096
-    // 356 / 74, 512^3 48 / 38), and at k = 16 its one step (1x16x4096 6.2 / 3.3).
-    if (k > 64 && (m * n <= 65536 || gx * gy < 64) && chain_fits(m, k, n)) {
-        if (ring_ok(variant, a, b, m, k, n)) {
-            switch (variant) {
-            case MM_AB: return launch_ring<MM_AB>(a, b, out, m, k, n, s);
-            case MM_ABT: return launch_ring<MM_ABT>(a, b, out, m, k, n, s);
-            case MM_ATB: return launch_ring<MM_ATB>(a, b, out, m, k, n, s);
-            default: break;
-            }
+    const Route r = route(variant, a, b, m, k, n);
+    if (r == ROUTE_MFMA) {
+        switch (variant) {
+        case MM_AB: return launch_mfma_ab(a, b, out, m, k, n, num_cus, s);
+        case MM_ABT: return launch_mfma_abt(a, b, out, m, k, n, num_cus, s);
+        case MM_ATB: return launch_mfma_atb(a, b, out, m, k, n, num_cus, s);
+        default: return fail(RQ_ERR_INVALID_ARGUMENT, "unknown matmul variant %d", variant);
         }
+    }
+    if (r == ROUTE_RING) return launch_ring(a, b, out, m, k, n, s);
+    if (r == ROUTE_CHAIN) {
         switch (variant) {
         case MM_AB: return launch_chain<MM_AB>(a, b, out, m, k, n, s);
         case MM_ABT: return launch_chain<MM_ABT>(a, b, out, m, k, n, s);
@@ -513,6 +513,7 @@ int launch_matmul_f32(int variant, const float *a, const float *b, float *out, i
         default: return fail(RQ_ERR_INVALID_ARGUMENT, "unknown matmul variant %d", variant);
         }
     }
+    const int64_t gx = cdiv(n, BN), gy = cdiv(m, BM);
     if (gx > 0x7fffffff || gy > 65535)
         return fail(RQ_ERR_SHAPE, "matmul grid too large (m=%lld n=%lld)", (long long)m, (long long)n);
     const dim3 grid((unsigned)gx, (unsigned)gy), block(TH);
@@ -527,15 +528,17 @@ int launch_matmul_f32(int variant, const float *a, const float *b, float *out, i
     return RQ_OK;
 }
 
-// C = A.B with A fp16 (exactly widened), where the register-staged chain
-// kernel serves the shape (few outputs, n <= 16, k > 64); RQ_ERR_UNSUPPORTED
-// (nothing launched) otherwise, and the caller widens A itself.
-int launch_matmul_f32_ah(const _Float16 *a, const float *b, float *out, int64_t m, int64_t k, int64_t n,
+// C = A.B with A fp16 (exactly widened) where the kernel of the shape loads
+// it as it is; RQ_ERR_UNSUPPORTED (nothing launched) otherwise, and the caller
+// widens A itself.
+int launch_matmul_f32_ah(const _Float16 *a, const float *b, float *out, int64_t m, int64_t k, int64_t n, int num_cus,
                          hipStream_t s) {
     if (m == 0 || n == 0) return RQ_OK;
-    const int64_t gx = cdiv(n, BN), gy = cdiv(m, BM);
-    if (!(k > 64 && (m * n <= 65536 || gx * gy < 64) && chain_fits(m, k, n)) || n > 16) return RQ_ERR_UNSUPPORTED;
-    return launch_chain<MM_AB, true>(a, b, out, m, k, n, s);
+    switch (route(MM_AB, a, b, m, k, n)) {
+    case ROUTE_MFMA: return launch_mfma_ab_f16(a, b, out, m, k, n, num_cus, s);
+    case ROUTE_CHAIN: return launch_chain<MM_AB, true>(a, b, out, m, k, n, s);
+    default: return RQ_ERR_UNSUPPORTED;
+    }
 }
 
 }  // namespace rq

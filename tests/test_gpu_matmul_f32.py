@@ -15,16 +15,14 @@ from rusty_amd import UnifiedTensor
 
 pytestmark = pytest.mark.gpu
 
-# Few outputs or few 64x64 tiles take the one-output-per-thread chain kernel
-# (k-chunks of 256 or 512 staged in LDS, column tiles of 8/16/32/64): k past
-# a chunk and not a multiple of 32, k = 0, every column-tile width; the others
-# (512x200x520, 1030x64x600) the 64x64 tiled kernel.  Both must match the
-# oracle bit for bit.
+# Products of a few k-steps take the 64x64 tiled kernel, A.B^T with few outputs
+# the ring chains, one 16x16 tile of outputs the register-staged chains, the
+# rest the matrix cores: k past a chunk and not a multiple of 32, k = 0, every
+# column-tile width.  All must match the oracle bit for bit.
 SHAPES = [(2, 2, 2), (1, 1024, 1024), (8, 1024, 1024), (65, 33, 70), (128, 256, 96), (3, 0, 5), (1, 4096, 4096),
           (1, 4097, 16), (5, 1000, 40), (33, 600, 9), (7, 300, 3), (2, 513, 100), (512, 4096, 16),
           (512, 200, 520), (1030, 64, 600),
-          # the DMA-ring chain kernel (16-byte rows, n > 16 or A.B^T): ragged row and
-          # column blocks with a partial last chunk, for all three variants
+          # 16-byte rows with ragged row and column blocks and a partial last chunk
           (20, 520, 44), (12, 700, 36)]
 
 
@@ -67,3 +65,60 @@ def test_shape_mismatch_raises(ctx, engine):
     out = UnifiedTensor.empty(ctx, [2, 5])
     with pytest.raises(ValueError):
         engine.matmul(ctx, A, B, out)
+
+
+# The matrix-core kernel's tiles (128x128, 64x64, 32x32, 16x64, 64x16): outputs
+# one short of, at and past whole tiles, k below a stage (32 or 64), at whole
+# stages and one past, row pitches in whole 16-byte pieces and not.
+MFMA_SHAPES = [(2050, 52, 2052), (1920, 64, 2047), (1023, 33, 1025), (1000, 96, 1000), (255, 100, 255),
+               (97, 65, 130), (64, 128, 64), (63, 127, 65), (15, 70, 1500), (16, 64, 4100), (1500, 70, 15),
+               (2100, 129, 16), (33, 17, 31), (17, 18, 19), (1, 20, 300), (300, 21, 1)]
+
+
+@pytest.mark.parametrize("m,k,n", MFMA_SHAPES)
+def test_matrix_core_tiles_bit_exact(ctx, engine, m, k, n):
+    test_matmul_family_bit_exact(ctx, engine, m, k, n)
+
+
+@pytest.mark.parametrize("k", [17, 30, 65])
+def test_padding_and_specials(ctx, engine, k):
+    """A partial last stage leaves every accumulator as it is: a sum that
+    underflowed to -0 keeps its sign, infinities and NaN stay in their rows
+    and columns, subnormals are kept."""
+    m, n = 70, 66
+    g = np.random.default_rng(k)
+    a = g.standard_normal((m, k), dtype=np.float32)
+    b = g.standard_normal((k, n), dtype=np.float32)
+    a[3], b[:, 5] = -1e-30, 1e-30  # outputs (3, 5): the products underflow to -0
+    a[7], b[:, 9] = 1e-42, np.float32(0.75)  # subnormal operands
+    a[11, 2], b[4, 13] = np.inf, np.nan
+    with np.errstate(all="ignore"):
+        want = orc.matmul(a, b, fused=True)
+        for op, x, y in (("matmul", a, b), ("matmul_bt", a, np.ascontiguousarray(b.T)),
+                         ("matmul_at", np.ascontiguousarray(a.T), b)):
+            got = _run(engine, ctx, op, x, y, m, n)
+            nan = np.isnan(want)
+            assert np.array_equal(np.isnan(got), nan)
+            assert np.array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+    assert np.signbit(want[3, 5]) and want[3, 5] == 0
+
+
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_unaligned_operands(ctx, engine, shift):
+    """Operands that start at any float (a view into a larger buffer)."""
+    m, k, n = 130, 72, 68
+    g = np.random.default_rng(shift)
+    a = g.standard_normal((m, k), dtype=np.float32)
+    b = g.standard_normal((k, n), dtype=np.float32)
+
+    def at(x):
+        t = UnifiedTensor.new(ctx, np.concatenate([np.zeros(shift, np.float32), x.ravel()]))
+        v = UnifiedTensor(ctx, t.ptr + 4 * shift, x.shape, t.dtype, owner=False)
+        v._base = t
+        return v
+
+    out = UnifiedTensor.empty(ctx, [m, n])
+    for op, x, y in (("matmul", a, b), ("matmul_bt", a, np.ascontiguousarray(b.T)),
+                     ("matmul_at", np.ascontiguousarray(a.T), b)):
+        getattr(engine, op)(ctx, at(x), at(y), out)
+        assert np.array_equal(out.to_vec().view(np.uint32), orc.matmul(a, b, fused=True).view(np.uint32))
