@@ -597,7 +597,7 @@ int rq_qmatmul_dx(rq_ctx *ctx, const rq_qweight *w, const void *dy, rq_dtype dy_
     if (!mul_ok(m, w->k_in, &t) || !mul_ok(m, w->n_out, &t)) return fail(RQ_ERR_SHAPE, "shape overflows");
     if (m == 0 || w->k_in == 0) return RQ_OK;
     if (!dx || (w->n_out > 0 && !dy)) return fail(RQ_ERR_INVALID_ARGUMENT, "null gradient pointer");
-    return launch_qmatmul_dx(*w, dy, dy_dtype, dx, dx_dtype, m, pick(ctx, stream));
+    return launch_qmatmul_dx(*w, dy, dy_dtype, dx, dx_dtype, m, ctx->num_cus, pick(ctx, stream));
 }
 
 }  // extern "C"

@@ -9,23 +9,32 @@
 // [out, in] orientation, so W is read as it lies, with no transpose.  The
 // weight gradient is not formed (the weight is frozen).
 //
-// Tiling: 64x64 output tiles per 256-thread block, 4x4 outputs per thread,
-// one f32 accumulator per output updated by fma in ascending n_out (the f32
+// One f32 accumulator per output updated by fma in ascending n_out (the f32
 // matmul family's order).  The weight tile is dequantized while it is staged
 // -- per-row codes f32(q) * s[row] (one rounding), affine codes
 // (f32(u) * s[g]) + b[g] (two roundings, no contraction), exactly the values
 // rq_qweight_dequantize writes -- so dX is bit-identical to the f32 matmul on
 // the dequantized weight without that weight ever existing in memory.
-// Memory: 1 B per weight element instead of 4.  Steps of 32 along n_out; the
-// next step's dY and code pieces are loaded into registers (8 codes and 8 dY
-// values per thread) before the current step's fmas run, so a block's loads
-// overlap its arithmetic (a few blocks per CU at prompt-sized m cannot hide
-// the latency by occupancy alone: 512 x 4096 x 4096 took 730 us with
-// single-buffered 16-step tiles).
+// Memory: 1 B per weight element instead of 4.
+//
+// k_dx_chain runs on the f32 matrix cores (mfma_chain.hpp) and serves every
+// call whose codes come in words (dx_chain_ok); k_qmatmul_dx, on the VALU,
+// the rest (k_in or n_out not a multiple of 4, unaligned operands, groups that
+// do not divide k_in).  Bound by the matrix instructions, which share the SIMD
+// with the dequantization (3-4 VALU instructions per element of a tile, for
+// 64 or 128 rows' products): us, VALU -> matrix cores, 512x4096x4096 affine 518 -> 140,
+// per-row 372 -> 139; 2048x4096x4096 affine 1616 -> 587; 16 rows x 11008x4096
+// 1144 -> 78 (the VALU kernel's 64x64 tiles left most CUs idle).
+//
+// k_qmatmul_dx: 64x64 output tiles per 256-thread block, 4x4 outputs per
+// thread, steps of 32 along n_out; the next step's dY and code pieces are
+// loaded into registers (8 codes and 8 dY values per thread) before the
+// current step's fmas run.
 #include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
+#include "mfma_chain.hpp"
 
 namespace rq {
 namespace {
@@ -164,6 +173,127 @@ __global__ __launch_bounds__(TH) void k_qmatmul_dx(const uint8_t *__restrict__ c
         }
 }
 
+// ---- the same product on the f32 matrix cores (mfma_chain.hpp) ----------------
+//
+// deq(W) as the chain product's B panel, rows along the outputs (k_in) and
+// the reduction over n_out: the codes of a piece (4 columns of one weight row)
+// are loaded as one word with the row's scale, or with the scale and bias of
+// the group the four columns share, and dequantized when the piece is staged,
+// to the bits rq_qweight_dequantize writes.  Served: codes 4-byte aligned with
+// k_in % 4 == 0, affine groups of a multiple of 4 dividing k_in (a group then
+// holds whole pieces, and row r's groups start at r k_in / group).
+template <int FMT, int R, int KC, int MF, int TILES, int TH_>
+struct PanelW : PanelOLds<R, KC, MF, TILES, TH_> {
+    using L = PanelOLds<R, KC, MF, TILES, TH_>;
+    static constexpr bool AFFINE = FMT == RQ_Q_AFFINE_U8;
+    struct Raw {
+        uint32_t c[L::NP];
+        float s[L::NP], b[AFFINE ? L::NP : 1];
+    };
+    struct Span {
+        ChainSpan c, s, b;
+    };
+    const uint8_t *codes;  // column c0 of row 0
+    const float *scales, *biases;
+    int64_t ld, left;  // codes per row; columns from c0 on
+    int gpr, group, c0;  // affine: groups per row; the panel's first column
+    __device__ __forceinline__ uint32_t code_records(int rows) const {
+        return rows > 0 ? (uint32_t)((rows - 1) * ld + left) : 0u;
+    }
+    __device__ __forceinline__ uint32_t scale_records(int rows) const {
+        return (uint32_t)(AFFINE ? rows * gpr : rows) * 4u;
+    }
+    __device__ __forceinline__ Span first(int64_t k) const {
+        const int rows = (int)(k < KC ? k : KC);
+        Span sp{{reinterpret_cast<uint64_t>(codes), code_records(rows)},
+                {reinterpret_cast<uint64_t>(scales), scale_records(rows)},
+                {reinterpret_cast<uint64_t>(biases), biases ? scale_records(rows) : 0u}};
+        return sp;
+    }
+    __device__ __forceinline__ void next(Span &sp, int st, int stages, int live) const {
+        sp.c.base += KC * ld;
+        sp.s.base += (AFFINE ? KC * (int64_t)gpr : KC) * 4;
+        if constexpr (AFFINE) sp.b.base += KC * (int64_t)gpr * 4;
+        if (st >= stages - 1) {
+            const int rows = st == stages - 1 ? live : 0;
+            sp.c.records = code_records(rows);
+            sp.s.records = scale_records(rows);
+            if constexpr (AFFINE) sp.b.records = biases ? scale_records(rows) : 0u;
+        }
+    }
+    struct Off {  // a lane's byte offsets of the pieces' codes and scales
+        uint32_t c[L::NP], s[L::NP];
+    };
+    __device__ __forceinline__ Off offsets(int t) const {
+        Off o;
+        const int col = c0 + 4 * (t % L::PR);
+#pragma unroll
+        for (int i = 0; i < L::NP; ++i) {
+            const int r = t / L::PR + L::STEP * i;
+            o.c[i] = (uint32_t)(r * ld + 4 * (t % L::PR));
+            o.s[i] = (uint32_t)(AFFINE ? r * gpr + col / group : r) * 4u;
+        }
+        return o;
+    }
+    __device__ __forceinline__ void load(Raw &raw, int i, const Span &sp, const Off &o) const {
+        raw.c[i] = __builtin_amdgcn_raw_buffer_load_b32(sp.c.rsrc(), o.c[i], 0, 0);
+        raw.s[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sp.s.rsrc(), o.s[i], 0, 0));
+        if constexpr (AFFINE)
+            raw.b[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sp.b.rsrc(), o.s[i], 0, 0));
+    }
+    __device__ __forceinline__ void stage(const Raw &raw, int i, float *lds, int t) const {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = deq1<FMT>((raw.c[i] >> (8 * e)) & 0xFFu, raw.s[i], raw.b[AFFINE ? i : 0]);
+        *reinterpret_cast<float4 *>(L::at(lds, i, t)) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+};
+
+template <int FMT, typename TY, int MF, int WM, int WN, int T, int KC, int MINB>
+__global__ __launch_bounds__(TH, MINB) void k_dx_chain(const uint8_t *__restrict__ codes,
+                                                       const float *__restrict__ scales,
+                                                       const float *__restrict__ biases, int group,
+                                                       const TY *__restrict__ dy, void *__restrict__ dx, bool dxf16,
+                                                       int64_t m, int64_t n_out, int64_t k_in, uint32_t rows, uint32_t cols) {
+    constexpr int TM = WM * T * MF, TN = WN * T * MF;
+    using PA = PanelK<TY, true, TM, KC, MF, T, TH>;
+    using PB = PanelW<FMT, TN, KC, MF, T, TH>;
+    using Tile = ChainTile<PA, PB, MF, WM, WN, T, T, KC, 1>;
+    __shared__ __attribute__((aligned(16))) float lds[Tile::LDS_FLOATS];
+    uint32_t tr, tc;
+    chain_tile_of(blockIdx.x, rows, cols, tr, tc);
+    const int64_t m0 = (int64_t)tr * TM, c0 = (int64_t)tc * TN;
+    PA pa;
+    pa.p = dy + m0 * n_out;
+    pa.ld = n_out;
+    pa.left = m - m0;
+    PB pb;
+    pb.codes = codes + c0;
+    pb.scales = scales;
+    pb.biases = biases;
+    pb.ld = k_in;
+    pb.left = k_in - c0;
+    pb.group = FMT == RQ_Q_AFFINE_U8 ? group : 1;
+    pb.gpr = FMT == RQ_Q_AFFINE_U8 ? (int)(k_in / group) : 0;
+    pb.c0 = (int)c0;
+    typename Tile::acc_t acc[T][T];
+    Tile::run(pa, pb, lds, n_out, threadIdx.x, acc);
+    Tile::each(acc, threadIdx.x, [&](int r, int c, float v) {
+        if (m0 + r < m && c0 + c < k_in) {
+            const int64_t o = (m0 + r) * k_in + c0 + c;
+            if (dxf16) static_cast<_Float16 *>(dx)[o] = (_Float16)v;
+            else static_cast<float *>(dx)[o] = v;
+        }
+    });
+}
+
+bool dx_chain_ok(const rq_qweight &w, const void *dy, rq_dtype dyt, int64_t m) {
+    const int64_t lim = (int64_t)1 << 29;
+    return aligned(w.codes, 4) && aligned(dy, dyt == RQ_F16 ? 8 : 16) && w.k_in % 4 == 0 && w.n_out % 4 == 0 &&
+           w.k_in * 64 < lim && w.n_out * 128 < lim && cdiv(m, 16) * cdiv(w.k_in, 16) < ((int64_t)1 << 31) &&
+           (w.format == RQ_Q_ROWWISE_I8 || (w.group % 4 == 0 && w.k_in % w.group == 0));
+}
+
 template <int FMT, bool DYF16>
 int launch_fmt(const rq_qweight &w, const void *dy, void *dx, bool dxf16, int64_t m, dim3 grid, hipStream_t s) {
     const uint8_t *codes = static_cast<const uint8_t *>(w.codes);
@@ -178,16 +308,43 @@ int launch_fmt(const rq_qweight &w, const void *dy, void *dx, bool dxf16, int64_
     return RQ_OK;
 }
 
+template <int FMT, typename TY>
+int launch_chain(const rq_qweight &w, const void *dyv, void *dx, bool dxf16, int64_t m, int num_cus, hipStream_t s) {
+    const ChainTiles t = chain_tiles(m, w.k_in, num_cus);
+    const dim3 grid((unsigned)(t.rows * t.cols));
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(TH), 0, s, static_cast<const uint8_t *>(w.codes), w.scales, w.biases,
+                           w.group, static_cast<const TY *>(dyv), dx, dxf16, m, w.n_out, w.k_in, (uint32_t)t.rows,
+                           (uint32_t)t.cols);
+    };
+    switch (t.shape) {
+    case CHAIN_128: go(k_dx_chain<FMT, TY, 32, 2, 2, 2, 32, 1>); break;
+    case CHAIN_64: go(k_dx_chain<FMT, TY, 32, 2, 2, 1, 32, 2>); break;
+    case CHAIN_32: go(k_dx_chain<FMT, TY, 16, 2, 2, 1, 64, 1>); break;
+    case CHAIN_16x64: go(k_dx_chain<FMT, TY, 16, 1, 4, 1, 64, 1>); break;
+    case CHAIN_64x16: go(k_dx_chain<FMT, TY, 16, 4, 1, 1, 64, 1>); break;
+    }
+    RQ_LAUNCH_CHECK();
+    return RQ_OK;
+}
+
 }  // namespace
 
 int launch_qmatmul_dx(const rq_qweight &w, const void *dy, rq_dtype dyt, void *dx, rq_dtype dxt, int64_t m,
-                      hipStream_t s) {
+                      int num_cus, hipStream_t s) {
+    const bool dyf16 = dyt == RQ_F16, dxf16 = dxt == RQ_F16;
+    if (dx_chain_ok(w, dy, dyt, m)) {
+        if (w.format == RQ_Q_ROWWISE_I8)
+            return dyf16 ? launch_chain<RQ_Q_ROWWISE_I8, _Float16>(w, dy, dx, dxf16, m, num_cus, s)
+                         : launch_chain<RQ_Q_ROWWISE_I8, float>(w, dy, dx, dxf16, m, num_cus, s);
+        return dyf16 ? launch_chain<RQ_Q_AFFINE_U8, _Float16>(w, dy, dx, dxf16, m, num_cus, s)
+                     : launch_chain<RQ_Q_AFFINE_U8, float>(w, dy, dx, dxf16, m, num_cus, s);
+    }
     const int64_t gx = cdiv(w.k_in, BN), gy = cdiv(m, BM);
     if (gx > 0x7fffffff || gy > 65535)
         return fail(RQ_ERR_SHAPE, "input-gradient grid too large (m=%lld k_in=%lld)", (long long)m,
                     (long long)w.k_in);
     const dim3 grid((unsigned)gx, (unsigned)gy);
-    const bool dyf16 = dyt == RQ_F16, dxf16 = dxt == RQ_F16;
     if (w.format == RQ_Q_ROWWISE_I8)
         return dyf16 ? launch_fmt<RQ_Q_ROWWISE_I8, true>(w, dy, dx, dxf16, m, grid, s)
                      : launch_fmt<RQ_Q_ROWWISE_I8, false>(w, dy, dx, dxf16, m, grid, s);

@@ -164,7 +164,7 @@ int launch_swiglu_generic(const rq_qweight &gate, const rq_qweight &up, const vo
 int launch_silu_mul(const void *g, const void *u, void *h, int64_t n, hipStream_t s);
 // dX[m, k_in] = dY[m, n_out] . deq(W), W dequantized while staged (f32 fma, ascending n_out).
 int launch_qmatmul_dx(const rq_qweight &w, const void *dy, rq_dtype dyt, void *dx, rq_dtype dxt, int64_t m,
-                      hipStream_t s);
+                      int num_cus, hipStream_t s);
 
 // Batched prompt kernels of the Llama runner (one launch each over n rows).
 // x[s] = f32(embed[tokens[s]]) for s < n.

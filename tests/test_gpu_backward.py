@@ -41,6 +41,34 @@ def test_dx_bit_exact_f32(ctx, engine, m, n_out, k_in, fmt):
     assert np.array_equal(bits(got), bits(want)), f"{np.count_nonzero(bits(got) != bits(want))} elements differ"
 
 
+@pytest.mark.parametrize("m,n_out,k_in,grp", [(2050, 36, 2052, 0), (1025, 100, 1028, 4), (130, 132, 64, 32),
+                                              (5, 1028, 1100, 0), (1100, 68, 12, 12), (33, 60, 256, 128),
+                                              (64, 64, 64, 64), (17, 30, 34, 0), (20, 40, 60, 24)])
+def test_dx_tiles_bit_exact(ctx, engine, m, n_out, k_in, grp):
+    """Every tile of the matrix-core kernel at ragged edges and partial last
+    stages, groups of one piece up, and the shapes it leaves to the VALU
+    kernel (widths not a multiple of 4, groups that do not divide k_in)."""
+    g = synth.rng(m + n_out + k_in)
+    if not grp:
+        q, s = synth.rowwise_weight(g, n_out, k_in)
+        w, wdeq = QuantizedTensor.rowwise(ctx, q, s), orc.rowwise_dequantize(q, s)
+    else:
+        u, s, b = synth.affine_weight(g, n_out, k_in, group=grp)
+        b = None if grp == 32 else b
+        w = QuantizedTensor.affine(ctx, u, s, b, group=grp)
+        wdeq = orc.affine_dequantize(u, s, np.zeros_like(s) if b is None else b, group=grp)
+    for dt in (np.float32, np.float16):
+        dy = g.standard_normal((m, n_out), dtype=np.float32).astype(dt)
+        want = orc.matmul(dy.astype(np.float32), wdeq.reshape(n_out, k_in), fused=True)
+        for out in (DType.FP32, DType.FP16):
+            dx = UnifiedTensor.empty(ctx, [m, k_in], out)
+            engine.qmatmul_dx(ctx, UnifiedTensor.new(ctx, dy), w, dx)
+            got = dx.to_vec()
+            ref = want if out is DType.FP32 else want.astype(np.float16)
+            assert np.array_equal(got.view(np.uint32 if out is DType.FP32 else np.uint16),
+                                  ref.view(np.uint32 if out is DType.FP32 else np.uint16))
+
+
 def test_dx_fp16(ctx, engine):
     g = synth.rng(5)
     q, s = synth.rowwise_weight(g, 768, 512)
