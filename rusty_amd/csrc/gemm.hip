@@ -124,13 +124,13 @@ __device__ __forceinline__ half8 u8x8_affine(uint2 w, float s, float c) {
 }
 
 // Tile order: consecutive blocks go round-robin to the 8 XCDs, so block b
-// runs on XCD b % 8; it takes position L = (b % 8) * (tiles / 8) + b / 8 of
-// a group-M order (GM m-tiles per group, n-tiles across, m fastest within a
+// runs on XCD b % 8; it takes position L = its XCD's first tile + b / 8 of
+// a group-M order (XCDs below tiles % 8 hold one tile more) (GM m-tiles per group, n-tiles across, m fastest within a
 // group).  The 32 concurrent tiles of one XCD then cover GM token panels x
 // 32/GM feature panels, so both X and W panels are reused in that XCD's L2.
 __device__ __forceinline__ void tile_of(int b, int tiles_m, int tiles_n, int gm, int &tm, int &tn) {
     const int tiles = tiles_m * tiles_n;  // b < tiles
-    const int L = (tiles % 8 == 0) ? (b % 8) * (tiles / 8) + b / 8 : b;
+    const int x = b % 8, L = x * (tiles / 8) + min(x, tiles % 8) + b / 8;
     const int per_group = gm * tiles_n;
     const int first_m = (L / per_group) * gm;
     const int gsize = min(gm, tiles_m - first_m);
@@ -152,8 +152,8 @@ __device__ __forceinline__ void tile_of(int b, int tiles_m, int tiles_n, int gm,
 // tn * BN/2 -- the gate (W, scales) in tile columns [0, BN/2), the up weight
 // (Wb, scalesb) in [BN/2, BN) -- and the epilogue writes h = silu(g) * u
 // (g and u rounded to fp16 first, as a separate silu*mul pass over stored
-// g and u would see them) to Yv, fp16 [M][I] (I % 8 == 0).  Only the two
-// large tiles are built with it (the smaller ones run near the SGPR limit).
+// g and u would see them) to Yv, fp16 [M][I] (I % 8 == 0).  Only the tiles of
+// 128 columns and more are built with it (the others run near the SGPR limit).
 // ROPE (BN = 64 = head_dim, per-row codes, no split): the tile's 64 features
 // are one head of the packed q/k/v output, and the epilogue applies the
 // rotary embedding to q and k heads -- o[d] = a c - b s, o[d + 32] = a s + b c
@@ -1024,48 +1024,130 @@ bool tile_fills(int64_t m, int64_t N, int64_t cus, int bm, int bn) {
     return bm <= std::max<int64_t>(64, m) && cdiv(m, bm) * cdiv(N, bn) * 3 >= 2 * cus;
 }
 
+// The tiles and what a launch on them takes, in us: `first` + per k-step of
+// 64 `step[t - 1]` with t tiles on every CU (t <= per_cu run together), plus
+// `next` for each further round.  Fitted on MI355X to grids of exactly 1, 2
+// and 3 tiles per CU at K = 1024 and 4096 (within 3 %); per-row codes, then
+// affine ones, whose expansion costs 1.2-1.5x per step.
+struct GemmTile {
+    int bm, bn, per_cu;
+    struct {
+        float first, next, step[3];
+    } cost[2];
+};
+enum { T128x256, T192x128, T128x128, T128x64, T64x128, T64x64, kTiles };
+constexpr GemmTile kTile[kTiles] = {
+    {128, 256, 1, {{9.2f, 8.0f, {0.81f}}, {6.4f, 4.0f, {1.02f}}}},
+    {192, 128, 1, {{5.5f, 4.0f, {0.685f}}, {5.4f, 4.0f, {0.825f}}}},
+    {128, 128, 1, {{6.3f, 4.0f, {0.47f}}, {4.4f, 3.0f, {0.654f}}}},
+    {128, 64, 1, {{6.5f, 4.0f, {0.275f}}, {6.4f, 5.0f, {0.35f}}}},
+    {64, 128, 2, {{4.4f, 1.0f, {0.298f, 0.55f}}, {4.2f, 2.0f, {0.38f, 0.70f}}}},
+    {64, 64, 3, {{4.2f, 1.0f, {0.173f, 0.31f, 0.48f}}, {4.4f, 1.0f, {0.256f, 0.415f, 0.61f}}}},
+};
+// Time of an m x N x 64 nk product on tile `id`.  A grid whose last round is
+// partly empty leaves power and bandwidth to the rest: 35 % of the empty
+// share comes back (2048x2560x2048 on 160 128x256 tiles 31.4 us where a full
+// round takes 35.1; 777x11008x4096 affine, 430 192x128 tiles, 101 of 114).
+double tile_cost(int id, int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus) {
+    const GemmTile &t = kTile[id];
+    const auto &c = t.cost[fmt];
+    const int64_t tiles = cdiv(m, t.bm) * cdiv(N, t.bn), per = cdiv(tiles, cus);
+    const int64_t full = per / t.per_cu, rem = per % t.per_cu;
+    const double us = c.first + (double)nk * (full * (double)c.step[t.per_cu - 1] + (rem ? c.step[rem - 1] : 0.0f)) +
+                      c.next * (double)(full + (rem > 0) - 1);
+    const double fill = (double)tiles / (double)(per * cus);
+    // 64x128 reads the most bytes per product beside 64x64: 8 % for operands
+    // and outputs that do not stay in the caches the fit had them in
+    return us * (1.0 - 0.35 * (1.0 - fill)) * (id == T64x128 ? 1.08 : 1.0);
+}
+
+// The largest tile whose grid still has >= 2/3 as many tiles as the device has
+// CUs, unless the fitted times say that another is at least 5 % faster: a
+// round of tiles that is nearly empty costs as much as a full one.  128x256
+// rather than 256x128 for the same outputs per block (one 128x64 wave tile
+// per wave): it stages 32 KiB per k-step instead of 40, in 256 cache lines
+// instead of 320 (2048x4096x4096 64.5 -> 62.1 us); 192x128 and 64x128 fill
+// the rounds between (us, before -> after: 2048x2560x2048 35.8 -> 25.3,
+// 1536x4096x4096 57.6 -> 49.3, 777x11008x4096 affine 117.5 -> 101.3; SwiGLU
+// pairs, with the down product, 300x5632x2048 59.1 -> 43.6, 128x5632x2048
+// 40.0 -> 25.9, 1536x5632x2048 148.5 -> 133.9; over 140 random shapes 0.95-1.74x).
+// 64x256 was never the best.  A 64x64 grid that would split K (launch_tiled) stays.
+int choose_tile(int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus) {
+    auto fills = [&](int id) { return tile_fills(m, N, cus, kTile[id].bm, kTile[id].bn); };
+    const int pick = fills(T128x256) ? T128x256 : fills(T128x128) ? T128x128 : fills(T128x64) ? T128x64 : T64x64;
+    if (pick == T64x64 && 4 * cdiv(m, 64) * cdiv(N, 64) <= 3 * cus) return pick;  // split K
+    int best = pick;
+    double us = tile_cost(pick, fmt, m, N, nk, cus) * 0.95;
+    for (int id = 0; id < kTiles; ++id) {
+        const double c = tile_cost(id, fmt, m, N, nk, cus);
+        if (c < us) {
+            best = id;
+            us = c;
+        }
+    }
+    return best;
+}
+
+// Gate and up as one grid (PAIR): the tiles of 128 columns and more, against
+// two products and the silu*mul pass over their results (about 3 us more
+// than the two): -1.
+int choose_pair_tile(int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus) {
+    auto fills = [&](int id) { return tile_fills(m, N, cus, kTile[id].bm, kTile[id].bn); };
+    const int pick = fills(T128x256) ? T128x256 : fills(T128x128) ? T128x128 : -1;
+    // two products of half the width; a split of K takes up to 8 blocks per tile
+    const int64_t I = N / 2, tiles = cdiv(m, 64) * cdiv(I, 64);
+    const int single = choose_tile(fmt, m, I, nk, cus);
+    double two;
+    if (single == T64x64 && 4 * tiles <= 3 * cus) {
+        const int64_t sp = std::max<int64_t>(1, std::min<int64_t>(nk / 8, 2 * tiles <= cus ? cus / tiles : 2));
+        const auto &c = kTile[T64x64].cost[fmt];
+        two = 2 * (c.first + (double)cdiv(nk, sp) * c.step[0] + 2.0);
+    } else {
+        two = 2 * tile_cost(single, fmt, m, I, nk, cus);
+    }
+    int best = pick;
+    double us = pick < 0 ? (two + 3.0) * 0.9 : tile_cost(pick, fmt, m, N, nk, cus) * 0.95;
+    for (int id : {T128x256, T192x128, T128x128, T64x128}) {
+        const double c = tile_cost(id, fmt, m, N, nk, cus);
+        if (c < us) {
+            best = id;
+            us = c;
+        }
+    }
+    return best;
+}
+
 // The fp16-activation GEMM over m rows, tile chosen by shape.
 int gemm_tiles(const rq_qweight &w, const float *scales, int fmt, const void *x, void *y, rq_dtype yt, int64_t m,
                int64_t cus, const GemmWorkspace &ws, hipStream_t s, const GemmPair &pair = GemmPair{},
                const float *xscale = nullptr) {
-    const int64_t N = w.n_out;
-    // The largest tile whose grid still has >= 2/3 as many tiles as the device
-    // has CUs: a block streams its X and W panels through one CU at a latency-
-    // bound rate, so a grid that leaves CUs idle loses more than smaller tiles
-    // cost.  Measured (N = K = 4096): m = 256 64x64 19.9 us (128x128: 36.2),
-    // m = 512 128x64 28.1 us (38.4), m = 768 128x128 39.0, m = 1536 256x128
-    // 61.2 us (128x128: 76.3); N = 11008, m = 256: 128x128 39.1 (64x64: 41.1).
     // Groups of 4 token panels per XCD and the ping-pong fragments beat
-    // token-major order and single buffering by 5-15 % at m = 2048.  The two
-    // large tiles run two k-groups of 4 waves with the weight staged in pairs
-    // of k-steps; 128x64 and 64x64 two k-groups of 2 waves, each wave all the
-    // tile's tokens (two groups of 4 waves there, each wave still expanding
+    // token-major order and single buffering by 5-15 % at m = 2048.  The tiles
+    // of 128 columns and more run two k-groups of 4 waves with the weight staged
+    // in pairs of k-steps; 128x64 and 64x64 two k-groups of 2 waves, each wave
+    // all the tile's tokens (two groups of 4 waves there, each wave still expanding
     // its W fragment for 1-2 MFMAs, measured 2-4 % slower than one group of 4
-    // and than these).  128x256 rather than 256x128: for the same outputs per block
-    // (one 128x64 wave tile per wave) it stages 32 KiB per k-step instead of
-    // 40, in 256 cache lines instead of 320 (2048x4096x4096 64.5 -> 62.1 us,
-    // N = 11008 176.4 -> 171.2, K = 11008 162.5 -> 156.9 us in one run), and
-    // it fills the device whenever 256x128 would.
-    // a tile taller than the tokens (rounded up to 64) only multiplies padding:
-    // 64 x 11008 x 4096 took 23.6 us on 128x64 tiles, 17.7 on split 64x64 ones
-    auto fills = [&](int bm, int bn) { return tile_fills(m, N, cus, bm, bn); };
-    if (pair.n_split) {  // gate and up: the two large tiles only (the caller falls back otherwise)
-        if (fills(128, 256))
-            return launch_tiled<128, 256, true, 4, 8, 4, 2, true, true>(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, pair);
-        if (fills(128, 128))
-            return launch_tiled<128, 128, true, 4, 8, 2, 2, true, true>(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, pair);
-        return RQ_ERR_UNSUPPORTED;
+    // and than these).
+    const int64_t N = w.n_out, nk = w.k_in / 64;
+    if (pair.n_split) {
+        switch (choose_pair_tile(fmt, m, N, nk, cus)) {
+        case T128x256: return launch_tiled<128, 256, true, 4, 8, 4, 2, true, true>(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, pair);
+        case T192x128: return launch_tiled<192, 128, true, 4, 8, 2, 2, true, true>(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, pair);
+        case T128x128: return launch_tiled<128, 128, true, 4, 8, 2, 2, true, true>(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, pair);
+        case T64x128: return launch_tiled<64, 128, true, 4, 8, 4, 2, true, true>(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, pair);
+        default: return RQ_ERR_UNSUPPORTED;  // the caller multiplies the two weights one after the other
+        }
     }
     const GemmPair np{};
-    if (fills(128, 256))
-        return launch_tiled<128, 256, true, 4, 8, 4, 2, true>(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, np, nullptr,
-                                                              xscale);
-    if (fills(128, 128))
-        return launch_tiled<128, 128, true, 4, 8, 2, 2, true>(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, np, nullptr,
-                                                              xscale);
-    if (fills(128, 64))
-        return launch_tiled<128, 64, true, 6, 4, 2, 2>(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, np, nullptr, xscale);
-    return launch_tiled<64, 64, true, 4, 4, 2, 2>(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, np, nullptr, xscale);
+    auto go = [&](auto launch) { return launch(w, scales, fmt, x, y, yt, m, 4, cus, ws, s, np, nullptr, xscale); };
+    switch (choose_tile(fmt, m, N, nk, cus)) {
+    case T128x256: return go(launch_tiled<128, 256, true, 4, 8, 4, 2, true>);
+    case T192x128: return go(launch_tiled<192, 128, true, 4, 8, 2, 2, true>);
+    case T128x128: return go(launch_tiled<128, 128, true, 4, 8, 2, 2, true>);
+    case T128x64: return go(launch_tiled<128, 64, true, 6, 4, 2, 2>);
+    case T64x128: return go(launch_tiled<64, 128, true, 4, 8, 4, 2, true>);
+    default: return go(launch_tiled<64, 64, true, 4, 4, 2, 2>);
+    }
 }
 
 }  // namespace
@@ -1085,15 +1167,16 @@ int gemm_tiles(const rq_qweight &w, const float *scales, int fmt, const void *x,
 // 128x128 tiles that each leave a third of the CUs idle) and g and u never
 // leave the block.  Weights of one shape, per-row int8 or affine u8 with
 // their load-time tables (rq_qweight_prepare, the same group), fp16
-// activations, I % 8 == 0; RQ_ERR_UNSUPPORTED otherwise, or when the grid is
-// too small for the two large tiles.
+// activations, I % 8 == 0; RQ_ERR_UNSUPPORTED otherwise, or when two products
+// (which split K over more blocks) are the faster way (choose_pair_tile).
 // A Llama layer's packed q/k/v projection with the rotary epilogue (see
 // k_gemm_rowwise, ROPE): q fp16 [m][n_heads][64] to q, k and v into the
 // caches at positions ro.p0 .. ro.p0 + m - 1.  Weights of (n_heads + 2 n_kv)
 // 64 rows, per-row int8 or affine u8 with the load-time table
-// (rq_qweight_prepare), fp16 x, and a token count whose tile choice is 64
-// wide (64x64 or 128x64); RQ_ERR_UNSUPPORTED (nothing launched) otherwise,
-// and the caller runs the product and the rotation separately.
+// (rq_qweight_prepare), fp16 x, and a shape for which a 64-wide tile (64x64 or
+// 128x64: one head per tile) is no slower than the best tile and a rotation
+// pass; RQ_ERR_UNSUPPORTED (nothing launched) otherwise, and the caller runs
+// the product and the rotation separately.
 int launch_gemm_qkv_rope(const rq_qweight &w, const _Float16 *x, int64_t m, const RopeOut &ro, _Float16 *q,
                          int num_cus, const GemmWorkspace &ws, hipStream_t s) {
     const int64_t N = w.n_out, K = w.k_in;
@@ -1105,10 +1188,15 @@ int launch_gemm_qkv_rope(const rq_qweight &w, const _Float16 *x, int64_t m, cons
         (int64_t)ro.p0 + m > ro.max_seq)
         return RQ_ERR_UNSUPPORTED;
     const int64_t cus = num_cus > 0 ? num_cus : 256;
-    if (tile_fills(m, N, cus, 128, 256) || tile_fills(m, N, cus, 128, 128)) return RQ_ERR_UNSUPPORTED;
     const float *sc = affine ? w.prep : w.scales;
     const int fmt = affine ? 1 : 0;
-    if (tile_fills(m, N, cus, 128, 64))
+    // the 64-wide tiles against the best tile and a rotation pass over its f32
+    // rows (6 bytes per value at ~4.5 TB/s, 2 us of launch)
+    const double a = tile_cost(T128x64, fmt, m, N, K / 64, cus), b = tile_cost(T64x64, fmt, m, N, K / 64, cus);
+    const double pass = 2.0 + 6e-6 / 4.5 * (double)m * (double)N;
+    if (std::min(a, b) > tile_cost(choose_tile(fmt, m, N, K / 64, cus), fmt, m, N, K / 64, cus) + pass)
+        return RQ_ERR_UNSUPPORTED;
+    if (a < b)
         return launch_tiled<128, 64, true, 6, 4, 2, 2>(w, sc, fmt, x, q, RQ_F16, m, 4, cus, ws, s, GemmPair{}, &ro);
     return launch_tiled<64, 64, true, 4, 4, 2, 2>(w, sc, fmt, x, q, RQ_F16, m, 4, cus, ws, s, GemmPair{}, &ro);
 }

@@ -324,6 +324,30 @@ def test_gemm_ragged(ctx, engine, m, n, k):
     assert ok, (max_abs, rel)
 
 
+# Every tile of the choice by fitted time (192x128 and 64x128 beside the power-of-two ones), with
+# a partial last row and column tile, k-steps odd and not a multiple of the ring period, both
+# formats and output types; rows at tile edges against the f64 truth.
+@pytest.mark.parametrize("m,n,k", [(1500, 4090, 128), (1345, 2300, 128), (1010, 4100, 1088), (600, 2600, 192),
+                                   (130, 4000, 2048), (250, 4100, 1088), (385, 3000, 320)])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_gemm_tile_choice(ctx, engine, m, n, k, fmt):
+    g = synth.rng(m + n + k + fmt)
+    if fmt:
+        u, s, b = synth.affine_weight(g, n, k)
+        w = QuantizedTensor.affine(ctx, u, s, b)
+    else:
+        (u, s), b = synth.rowwise_weight(g, n, k), None
+        w = QuantizedTensor.rowwise(ctx, u, s)
+    x = synth.activations(g, m, k, sigma=0.5)
+    rows = np.unique(np.r_[0, 1, np.minimum(np.arange(63, m, 64), m - 1), m - 2, m - 1])
+    truth = orc.qlinear_truth(u, s, b, x[rows].astype(np.float32), fmt)
+    for ydt in (np.float16, np.float32):
+        y = qmm(ctx, engine, w, x, ydt)
+        assert np.isfinite(y).all()
+        max_abs, rel, ok = f16_tol_check(y[rows], truth)
+        assert ok, (ydt, max_abs, rel)
+
+
 # Split-K (tile grids covering at most half of a 256-CU device): 17 and 64 tokens at 4096x4096
 # (64 tiles of 64x64, 4 splits of 16 k-steps), 30 tokens at 1000x11008 (16 tiles, 16 splits of
 # 11 k-steps, the last of 7), 100 tokens at 1000x1088 (32 tiles; 17 k-steps allow 2 splits of at

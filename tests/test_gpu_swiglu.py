@@ -167,6 +167,35 @@ def test_swiglu_prefill_fused_affine(ctx, engine, m, inter, hidden):
     assert ok
 
 
+@pytest.mark.parametrize("m,inter,hidden", [(17, 264, 128), (65, 1000, 128), (300, 1000, 192), (577, 1032, 128),
+                                            (1400, 2000, 64)])
+def test_swiglu_prefill_fused_tiles(ctx, engine, m, inter, hidden):
+    """The fused gate/up product on the 64x128 and 192x128 tiles with partial
+    last tiles (in rows, and in the columns of both halves): h at tile-edge
+    rows against the f64 truth, both weight formats."""
+    g = synth.rng(77 + m)
+    x = synth.activations(g, m, hidden, sigma=0.5)
+    rows = np.unique(np.r_[0, 1, np.minimum(np.arange(63, m, 64), m - 1), m - 1])
+    wg, sg, wu, su, wd, sd = weights(g, inter, hidden)
+    _, h = run_mlp(ctx, engine, x, wg, sg, wu, su, wd, sd, ydt=np.float32)
+    _, _, ok = f16_tol_check(h[rows], h_truth(x[rows], wg, sg, wu, su))
+    assert ok and np.isfinite(h).all()
+    ug, sg, bg = synth.affine_weight(g, inter, hidden)
+    uu, su, bu = synth.affine_weight(g, inter, hidden)
+    G, U = QuantizedTensor.affine(ctx, ug, sg, bg), QuantizedTensor.affine(ctx, uu, su, bu)
+    D = QuantizedTensor.rowwise(ctx, wd, sd)
+    Y = UnifiedTensor.empty(ctx, [m, hidden], DType.FP32)
+    ha = engine.mlp_swiglu(ctx, UnifiedTensor.new(ctx, x, dtype=DType.FP16), G, U, D, Y)
+    ha = ha.to_vec().reshape(-1)[: m * inter].reshape(m, inter)
+    xr = x[rows].astype(np.float32)
+    gt = orc.qlinear_truth(ug, sg, bg, xr, 1).astype(np.float16).astype(np.float64)
+    ut = orc.qlinear_truth(uu, su, bu, xr, 1).astype(np.float16).astype(np.float64)
+    with np.errstate(over="ignore"):
+        ht = gt / (1.0 + np.exp(-gt)) * ut
+    _, _, ok = f16_tol_check(ha[rows], ht)
+    assert ok and np.isfinite(ha).all()
+
+
 def test_swiglu_prefill_fused_128x128(ctx, engine):
     """1024 tokens x 2 x 2048 rows take the fused epilogue on the 128x128 tile
     (the cases above run 128x256): h and y against the f64 truth on rows at
