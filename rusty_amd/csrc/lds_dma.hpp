@@ -1,5 +1,5 @@
 // Buffer resources and global -> LDS DMA for gfx950 (CDNA4), shared by the
-// kernels that stage operands through LDS rings (gemm.hip, matmul_f32.hip).
+// kernels that stage operands through LDS rings (gemm.hip, matmul_f32.hip, prefill.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -41,7 +41,7 @@ __device__ __forceinline__ uint32_t lds_addr(T *p) {
 // base (one wait state before the load, as the ISA requires).  The compiler
 // reserves M0 and warns that the "m0" clobber is not honoured (-Winline-asm):
 // that is safe only while nothing else in these kernels holds a value in M0
-// across a DMA, and in the device assembly of gemm.hip and matmul_f32.hip the
+// across a DMA, and in the device assembly of gemm.hip, matmul_f32.hip and prefill.hip the
 // only instructions naming M0 are these moves (each directly before its load).
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint32_t lds_addr, uint32_t voff) {
     const uint32_t l = __builtin_amdgcn_readfirstlane(lds_addr);

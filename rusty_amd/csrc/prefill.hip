@@ -9,9 +9,11 @@
 //                       q to an fp16 [S][n_heads][hd] buffer, k and v (fp16)
 //                       into the KV cache at positions p0..p0+S-1
 //   k_attn_prefill      causal GQA attention of the S queries over cache
-//                       positions 0..p0+S-1 on the matrix cores
+//                       positions 0..p0+S-1 on the matrix cores (short chunks)
+//   k_attn_prefill_rows the same for chunks that fill the device with blocks
+//                       of 128 queries
 //
-// Attention (flash-style, four waves per (query tile of 32, head)):
+// Attention of short chunks (flash-style, four waves per (query tile of 32, head)):
 // the scores of a key tile are computed transposed, S^T = K . Q^T, with
 // v_mfma_f32_32x32x16_f16: A = 32 cache rows of K (lane l: row l % 32, the
 // 8 halves 16 s + 8 (l / 32) of k-step s -- one 16-byte load), B = Q^T (the
@@ -28,6 +30,7 @@
 // accumulators are f32 (exponentials as 2^x on scores scaled by log2 e);
 // q, k, v and p enter the matrix cores as fp16.
 #include "common.hpp"
+#include "lds_dma.hpp"
 
 namespace rq {
 namespace {
@@ -39,9 +42,6 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00020000);
-}
 __device__ __forceinline__ uint4 bload(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
     return make_uint4(v.x, v.y, v.z, v.w);
@@ -342,6 +342,203 @@ __global__ __launch_bounds__(NW * 64) void k_attn_prefill(const _Float16 *__rest
     }
 }
 
+// The same attention for chunks long enough to fill the device with blocks
+// of 128 queries: four waves of 32 consecutive queries of one head walk the
+// same key tiles of 64, which pass through LDS once per block (DMA, a ring of
+// three stages, one barrier per tile) instead of once per 32 queries through
+// every wave's registers.  K fragments are 16-byte reads of swizzled rows; V^T
+// fragments come from the row-major V tile by transposing reads
+// (ds_read_b64_tr_b16: 16 lanes take a block of 4 keys x 16 dims and each gets
+// one dim's 4 keys), in the key order the score accumulators hold P in.
+// The softmax is what bounds it: per score one max, one fma into the exponent,
+// one quarter-rate exp2, one add and half a conversion, against 16 matrix
+// instructions per 64 keys (counters at 2048 queries after 2048 cached
+// positions: VALU issuing 76 % of the cycles, matrix cores 28 %).  So the rest
+// is kept off every tile: scale and maximum enter the exponent's fma, the mask
+// runs on a wave's last tile only, and the accumulators are rescaled only when
+// some query's maximum passed the one they are relative to by 2^8 (P then
+// reaches 256, in fp16 to the same relative precision; sums are f32).
+// 4096 positions in two chunks, 32 heads of 64, per layer: 304 -> 120 us (573
+// TFLOP/s of the causal work).
+template <int HD>
+__global__ __launch_bounds__(256, 2) void k_attn_prefill_rows(const _Float16 *__restrict__ q, const _Float16 *__restrict__ kc,
+                                                           const _Float16 *__restrict__ vc, _Float16 *__restrict__ out,
+                                                           int p0, int n, int n_heads, int n_kv, int max_seq) {
+    constexpr int KS = HD / 16, DT = HD / 32;
+    constexpr int ROW = HD * 2, CH = ROW / 16;  // bytes and 16-byte chunks per row
+    constexpr int KT = 64, NS = 3;
+    constexpr int TILE = KT * ROW;                   // one operand's tile
+    constexpr int UW = TILE / 1024 / 4;              // DMA units per wave and operand
+    constexpr int RPU = 1024 / ROW;                  // rows per unit
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[NS * 2 * TILE];
+    const int nqb = (n + 127) / 128;
+    const int head = blockIdx.x % n_heads;
+    const int qb = (nqb - 1 - (int)blockIdx.x / n_heads) * 128;  // the longest first
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 31, hf = lane >> 5;
+    const int q0 = qb + 32 * wv;
+    const int g = head / (n_heads / n_kv);
+    const int kv_len = p0 + n;
+    const auto rk = make_rsrc_s(kc + (size_t)g * max_seq * HD, (uint32_t)kv_len * ROW);
+    const auto rv = make_rsrc_s(vc + (size_t)g * max_seq * HD, (uint32_t)kv_len * ROW);
+    const auto rq = make_rsrc_s(q, (uint32_t)n * n_heads * ROW);
+
+    // LDS chunk c of row r holds global chunk c ^ f(r): K so that 16 rows at one
+    // chunk, V so that 4 rows x 4 chunks, cover the banks
+    auto fk = [](int r) { return HD == 64 ? (r >> 1) & 7 : r & 15; };
+    auto fv = [](int r) { return HD == 64 ? ((r >> 1) & 1) << 2 : (r & 3) << 2; };
+    uint32_t koff[UW], voff[UW];
+#pragma unroll
+    for (int u = 0; u < UW; ++u) {
+        const int r = (wv * UW + u) * RPU + lane / CH, c = lane % CH;
+        koff[u] = (uint32_t)(r * ROW + ((c ^ fk(r)) * 16));
+        voff[u] = (uint32_t)(r * ROW + ((c ^ fv(r)) * 16));
+    }
+    const int last_b = min(p0 + qb + 127, kv_len - 1);
+    const int ntiles = last_b / KT + 1;                                 // of the block
+    const int mine = q0 < n ? min(p0 + q0 + 31, kv_len - 1) / KT + 1 : 0;  // of this wave
+    const uint32_t lds0 = lds_addr(&lds[0]);
+    auto dma = [&](int kt) {
+        const bool live = kt < ntiles;
+        const uint32_t base = lds0 + (uint32_t)(kt % NS) * (2 * TILE) + (uint32_t)(wv * UW) * 1024u;
+#pragma unroll
+        for (int u = 0; u < UW; ++u) {
+            dma16(rk, base + (uint32_t)u * 1024u, live ? koff[u] + (uint32_t)kt * TILE : kOOB);
+            dma16(rv, base + (uint32_t)TILE + (uint32_t)u * 1024u, live ? voff[u] + (uint32_t)kt * TILE : kOOB);
+        }
+    };
+    half8 qf[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        const uint32_t off = q0 + col < n ? (((uint32_t)(q0 + col) * n_heads + head) * HD + 16 * s + 8 * hf) * 2u : kOOB;
+        qf[s] = __builtin_bit_cast(half8, bload(rq, off));
+    }
+    dma(0);
+    dma(1);
+    const int qpos = p0 + q0 + col;
+    // scores in log2 units (see above): p = 2^(c s - c m)
+    const float c = 1.4426950408889634f / sqrtf((float)HD);
+    float m_run = -__builtin_inff(), l_run = 0.0f;
+    floatx16 o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+    // LDS byte offsets of this lane's reads within a tile
+    uint32_t ka[KS], va[DT][2];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) ka[s] = (uint32_t)(col * ROW + (((2 * s + hf) ^ fk(col)) * 16));
+    const int i16 = lane & 15, kr = 4 * hf + i16 / 4;  // V: the lane's key row of a block of 4 (and 8 rows on)
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int r = kr + 8 * e, ch = 4 * d + 2 * ((lane >> 4) & 1) + (i16 & 3) / 2;
+            va[d][e] = (uint32_t)(r * ROW + ((ch ^ fv(r)) * 16) + (i16 & 1) * 8);
+        }
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) short4v lds_short4;
+    typedef __attribute__((address_space(3))) half8 lds_half8;
+    struct Scores {
+        floatx16 t[2];  // [t][r]: key 64 kt + 32 t + 8 (r / 4) + 4 hf + r % 4 against query qpos
+    };
+    auto scores = [&](int kt, Scores &sc) {
+        const uint32_t kb = lds0 + (uint32_t)(kt % NS) * (2 * TILE);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc.t[t][r] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const lds_half8 *kp = (const lds_half8 *)(kb + ka[s]);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                sc.t[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kp[t * 32 * ROW / 16], qf[s], sc.t[t], 0, 0, 0);
+        }
+    };
+    auto weigh = [&](int kt, Scores &sc) {  // softmax and P . V of tile kt
+        const uint32_t vb = lds0 + (uint32_t)(kt % NS) * (2 * TILE) + TILE;
+        if (kt == mine - 1) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int key = KT * kt + 32 * t + 8 * (r >> 2) + 4 * hf + (r & 3);
+                    sc.t[t][r] = key <= qpos ? sc.t[t][r] : -__builtin_inff();
+                }
+        }
+        float mt = sc.t[0][0];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sc.t[t][r]);
+        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        if (__builtin_amdgcn_ballot_w64((mt - m_run) * c > 8.0f)) {
+            const float m_new = fmaxf(m_run, mt);
+            const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * c);
+            m_run = m_new;
+            l_run *= alpha;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+        }
+        const float mc = m_run * c;
+        half8 pf[4];
+        float ls[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc.t[t][r], c, -mc));
+                ls[r & 1] += pr;
+                pf[2 * t + (r >> 3)][r & 7] = (_Float16)pr;
+            }
+        l_run += ls[0] + ls[1];
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+            lds_short4 *pa = (lds_short4 *)(vb + va[d][0]), *pb = (lds_short4 *)(vb + va[d][1]);
+#pragma unroll
+            for (int s2 = 0; s2 < 4; ++s2) {
+                const short4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(pa + s2 * 16 * ROW / 8);
+                const short4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16(pb + s2 * 16 * ROW / 8);
+                const uint2 ua = __builtin_bit_cast(uint2, a), ub = __builtin_bit_cast(uint2, b);
+                const half8 vf = __builtin_bit_cast(half8, make_uint4(ua.x, ua.y, ub.x, ub.y));
+                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[s2], o[d], 0, 0, 0);
+            }
+        }
+    };
+    // The scores of tile kt + 1 are multiplied while tile kt's softmax runs.
+    Scores sc[2];
+    wait_vmcnt<2 * UW>();
+    __syncthreads();
+    if (mine > 0) scores(0, sc[0]);
+    for (int kt = 0; kt < ntiles; kt += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            // tile kt + u + 1 has landed, and every wave is done with tile kt + u - 1
+            wait_vmcnt<0>();
+            __syncthreads();
+            dma(kt + u + 2);
+            if (kt + u + 1 < mine) scores(kt + u + 1, sc[1 - u]);
+            if (kt + u < mine) weigh(kt + u, sc[u]);
+        }
+    }
+    wait_vmcnt<0>();  // no DMA in flight past this point
+    if (q0 + col >= n) return;
+    const float inv = 1.0f / (l_run + __shfl_xor(l_run, 32));
+    _Float16 *orow = out + ((size_t)(q0 + col) * n_heads + head) * HD;
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            const half4 v = {(_Float16)(o[d][4 * r4] * inv), (_Float16)(o[d][4 * r4 + 1] * inv),
+                             (_Float16)(o[d][4 * r4 + 2] * inv), (_Float16)(o[d][4 * r4 + 3] * inv)};
+            *reinterpret_cast<half4 *>(orow + 32 * d + 8 * r4 + 4 * hf) = v;
+        }
+}
+
 }  // namespace
 
 int launch_embed_rows(const int *tokens, const _Float16 *embed, int H, float *x, int n, hipStream_t s) {
@@ -377,6 +574,21 @@ int launch_rope_scatter(const float *qkv, const float2 *rope, int p0, int n, int
 int launch_attn_prefill(const _Float16 *q, const _Float16 *kc, const _Float16 *vc, _Float16 *out, int p0, int n,
                         int n_heads, int n_kv, int hd, int max_seq, hipStream_t s) {
     if (p0 % 32 != 0 || n < 1 || (hd != 64 && hd != 128) || n_heads % n_kv != 0) return RQ_ERR_UNSUPPORTED;
+    // Blocks of 128 queries from three quarters of a 256-CU device on (us for
+    // three layers' attention and the rest of a 4-layer 1.1B-shape prompt, small
+    // blocks -> these: 768 positions 542 -> 529, 1024 628 -> 615, 2048 1047 ->
+    // 939, 4096 2388 -> 1942; 512, 128 blocks, 389 -> 397).
+    const int blocks = n_heads * ((n + 127) / 128);
+    if (blocks >= 192) {
+        if (hd == 64)
+            hipLaunchKernelGGL((k_attn_prefill_rows<64>), dim3((unsigned)blocks), dim3(256), 0, s, q, kc, vc, out, p0,
+                               n, n_heads, n_kv, max_seq);
+        else
+            hipLaunchKernelGGL((k_attn_prefill_rows<128>), dim3((unsigned)blocks), dim3(256), 0, s, q, kc, vc, out, p0,
+                               n, n_heads, n_kv, max_seq);
+        RQ_LAUNCH_CHECK();
+        return RQ_OK;
+    }
     const dim3 grid((unsigned)(n_heads * ((n + 31) / 32)));
     if (hd == 64)
         hipLaunchKernelGGL((k_attn_prefill<64, 4>), grid, dim3(256), 0, s, q, kc, vc, out, p0, n, n_heads, n_kv,

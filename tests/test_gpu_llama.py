@@ -324,6 +324,30 @@ def _check_steps_pick(dec, ties):
             assert np.count_nonzero(lg == lg.max()) >= 2, (i, lg.max())
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd,prompt,rows", [(16, 4, 64, 1555, 2048), (16, 2, 64, 3107, 1536),
+                                                         (16, 16, 128, 1601, 2048)])
+@pytest.mark.parametrize("sharp", [1.0, 25.0])
+def test_prefill_attention_of_long_chunks(ctx, n_heads, n_kv, hd, prompt, rows, sharp):
+    """Chunks of enough positions for the 128-query blocks of the prefill
+    attention (a partial last block, a second chunk behind 1536 cached
+    positions): the last position's logits against the oracle.  Its value
+    depends on every row of the first layer's attention.  `sharp` scales the
+    query projection, so that scores spread over many powers of two and the
+    running maximum rises in steps larger than the kernel's rescaling
+    threshold."""
+    cfg = LlamaConfig(n_layers=2, hidden=n_heads * hd, n_heads=n_heads, n_kv_heads=n_kv, head_dim=hd,
+                      intermediate=256, vocab=96, max_seq=-(-(prompt + 2) // 32) * 32)
+    w = synth_weights(cfg, seed=prompt)
+    for layer in w.layers:
+        layer["q"] = (layer["q"][0], layer["q"][1] * np.float32(sharp))
+    tokens = np.random.default_rng(prompt).integers(0, cfg.vocab, prompt)
+    r = LlamaRunner(ctx, cfg, w)
+    r.set_prefill(min(rows, -(-cfg.max_seq // 32) * 32, 2048))
+    r.prefill(tokens)
+    toks = r.tokens()
+    check_steps(cfg, w, toks, r.logits()[None], prompt, 1e-2 if sharp == 1.0 else 2e-2, f"long {prompt} x{sharp}")
+
+
 def test_greedy_pick_ties_and_threshold(ctx):
     """top_k with k = 1 as the reference scans (kernels.wgsl:173-188): the first
     index among equal maxima, and index 0 when no logit exceeds -1e9."""
