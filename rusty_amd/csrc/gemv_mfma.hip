@@ -116,17 +116,40 @@ __device__ __forceinline__ half8 u8x8_exact(uint32_t lo, uint32_t hi) {
 
 // 8 f32 values x, scaled by 2^-sh (SC; exact) -> hi = fp16(x), lo =
 // fp16(x - hi) (round to nearest even): hi + lo equals x to about 2^-22
-// relative while |x| stays inside fp16's range.
-template <bool SC = false>
+// relative while |x| stays inside fp16's range.  Every block splits all of X.
+// PAIR: pairs are converted by one v_cvt_pk_f16_f32 and the residual is taken
+// from that pair, three instructions per value; written by value, the compiler
+// converts each one a second time, alone, for the residual.  Same bits.  Per-row
+// codes take it (us, by value -> by pairs: m = 3 / 8 11008 x 4096 17.64 ->
+// 16.92, 20.30 -> 19.50; 4096 x 11008 17.66 -> 16.54, 18.86 -> 18.29; 4096^2 m = 4
+// 7.98 -> 7.84); affine codes, whose four scale and bias vectors leave the
+// registers full, do not (m = 3 / 8 11008 x 4096 27.08 -> 28.93, 29.33 -> 30.89;
+// 4096^2 m = 13 12.27 -> 12.53).
+template <bool SC, bool PAIR>
 __device__ __forceinline__ void f32x8_split(const uint4 a, const uint4 b, half8 &hi, half8 &lo, int sh = 0) {
+    typedef float f2_t __attribute__((ext_vector_type(2)));
     float f[8] = {__builtin_bit_cast(float, a.x), __builtin_bit_cast(float, a.y), __builtin_bit_cast(float, a.z),
                   __builtin_bit_cast(float, a.w), __builtin_bit_cast(float, b.x), __builtin_bit_cast(float, b.y),
                   __builtin_bit_cast(float, b.z), __builtin_bit_cast(float, b.w)};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        if constexpr (SC) f[e] = __builtin_amdgcn_ldexpf(f[e], -sh);
-        hi[e] = (_Float16)f[e];
-        lo[e] = (_Float16)(f[e] - (float)hi[e]);
+    for (int e = 0; e < 8; e += 2) {
+        if constexpr (SC) {
+            f[e] = __builtin_amdgcn_ldexpf(f[e], -sh);
+            f[e + 1] = __builtin_amdgcn_ldexpf(f[e + 1], -sh);
+        }
+        if constexpr (PAIR) {
+            const h2_t h = __builtin_convertvector((f2_t{f[e], f[e + 1]}), h2_t);
+            const h2_t l = __builtin_convertvector((f2_t{f[e] - (float)h.x, f[e + 1] - (float)h.y}), h2_t);
+            hi[e] = h.x;
+            hi[e + 1] = h.y;
+            lo[e] = l.x;
+            lo[e + 1] = l.y;
+        } else {
+            hi[e] = (_Float16)f[e];
+            lo[e] = (_Float16)(f[e] - (float)hi[e]);
+            hi[e + 1] = (_Float16)f[e + 1];
+            lo[e + 1] = (_Float16)(f[e + 1] - (float)hi[e + 1]);
+        }
     }
 }
 
@@ -339,7 +362,7 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mfma(const int8_t *__restrict
                             const int j = 2 * gi + jj;
                             const half8 ue = u8x8_exact(a[j].x, a[j].y);
                             half8 hi, lo;
-                            f32x8_split<SC>(b.x[2 * j], b.x[2 * j + 1], hi, lo, sh);
+                            f32x8_split<SC, false>(b.x[2 * j], b.x[2 * j + 1], hi, lo, sh);
                             tg = __builtin_amdgcn_mfma_f32_16x16x32_f16(ue, hi, tg, 0, 0, 0);
                             tg = __builtin_amdgcn_mfma_f32_16x16x32_f16(ue, lo, tg, 0, 0, 0);
                             xg = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, hi, xg, 0, 0, 0);
@@ -364,7 +387,7 @@ __global__ __launch_bounds__(NWV * 64) void k_gemv_mfma(const int8_t *__restrict
                     for (int j = 0; j < 8; ++j) {
                         const half8 av = i8x8_to_half8(a[j].x, a[j].y);
                         half8 hi, lo;
-                        f32x8_split<SC>(b.x[2 * j], b.x[2 * j + 1], hi, lo, sh);
+                        f32x8_split<SC, true>(b.x[2 * j], b.x[2 * j + 1], hi, lo, sh);
                         t = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, hi, t, 0, 0, 0);
                         t = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, lo, t, 0, 0, 0);
                     }
