@@ -1088,14 +1088,21 @@ int choose_tile(int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus) {
     return best;
 }
 
+// The copy-out of a PAIR tile addresses bm rows of h (I fp16 values each) with
+// 32-bit offsets and masks the pieces past a row with kOOB = 2^31, which must
+// lie past the tile's rows: the taller the tile, the narrower the h it serves.
+bool pair_fits(int id, int64_t I) { return kTile[id].bm * I * 2 < (int64_t)kOOB; }
+
 // Gate and up as one grid (PAIR): the tiles of 128 columns and more, against
 // two products and the silu*mul pass over their results (about 3 us more
 // than the two): -1.
 int choose_pair_tile(int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus) {
+    const int64_t I = N / 2;
+    if (!pair_fits(T128x256, I)) return -1;
     auto fills = [&](int id) { return tile_fills(m, N, cus, kTile[id].bm, kTile[id].bn); };
     const int pick = fills(T128x256) ? T128x256 : fills(T128x128) ? T128x128 : -1;
     // two products of half the width; a split of K takes up to 8 blocks per tile
-    const int64_t I = N / 2, tiles = cdiv(m, 64) * cdiv(I, 64);
+    const int64_t tiles = cdiv(m, 64) * cdiv(I, 64);
     const int single = choose_tile(fmt, m, I, nk, cus);
     double two;
     if (single == T64x64 && 4 * tiles <= 3 * cus) {
@@ -1108,6 +1115,7 @@ int choose_pair_tile(int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus) {
     int best = pick;
     double us = pick < 0 ? (two + 3.0) * 0.9 : tile_cost(pick, fmt, m, N, nk, cus) * 0.95;
     for (int id : {T128x256, T192x128, T128x128, T64x128}) {
+        if (!pair_fits(id, I)) continue;
         const double c = tile_cost(id, fmt, m, N, nk, cus);
         if (c < us) {
             best = id;
@@ -1211,8 +1219,7 @@ int launch_gemm_swiglu(const rq_qweight &gate, const rq_qweight &up, const void 
         return RQ_ERR_UNSUPPORTED;
     if ((!affine && (gate.format != RQ_Q_ROWWISE_I8 || up.format != RQ_Q_ROWWISE_I8)) || up.n_out != I || up.k_in != K ||
         xt != RQ_F16 || I % 8 != 0 || K % 64 != 0 || K > (1 << 21) || !aligned(gate.codes, 16) ||
-        !aligned(up.codes, 16) || !aligned(x, 16) || !aligned(h, 16) || m > 0x7fffffff || 2 * I > 0x7fffffff ||
-        128 * I * 2 >= (1ll << 31))
+        !aligned(up.codes, 16) || !aligned(x, 16) || !aligned(h, 16) || m > 0x7fffffff || 2 * I > 0x7fffffff)
         return RQ_ERR_UNSUPPORTED;
     rq_qweight w = gate;
     w.n_out = 2 * I;
@@ -1291,3 +1298,14 @@ int launch_gemm(const rq_qweight &w, const void *x, rq_dtype xt, void *y, rq_dty
 }
 
 }  // namespace rq
+
+// For the tests, no part of the C ABI: the tile (bm * 1000 + bn) that the
+// fp16-activation GEMM takes for an m x n_out x k_in product (fmt 0: per-row
+// codes, 1: affine), or with `pair` for SwiGLU's gate and up of n_out rows
+// each; -1 where the two are multiplied one after the other.  Host arithmetic.
+extern "C" int rusty_gemm_tile(int fmt, int64_t m, int64_t n_out, int64_t k_in, int num_cus, int pair) {
+    using namespace rq;
+    const int id = pair ? choose_pair_tile(fmt, m, 2 * n_out, k_in / 64, num_cus)
+                        : choose_tile(fmt, m, n_out, k_in / 64, num_cus);
+    return id < 0 ? -1 : kTile[id].bm * 1000 + kTile[id].bn;
+}
