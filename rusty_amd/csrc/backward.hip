@@ -287,11 +287,14 @@ __global__ __launch_bounds__(TH, MINB) void k_dx_chain(const uint8_t *__restrict
     });
 }
 
-bool dx_chain_ok(const rq_qweight &w, const void *dy, rq_dtype dyt, int64_t m) {
+bool dx_chain_ok(const rq_qweight &w, const void *dy, rq_dtype dyt, int64_t m, int num_cus) {
     const int64_t lim = (int64_t)1 << 29;
-    return aligned(w.codes, 4) && aligned(dy, dyt == RQ_F16 ? 8 : 16) && w.k_in % 4 == 0 && w.n_out % 4 == 0 &&
-           w.k_in * 64 < lim && w.n_out * 128 < lim && cdiv(m, 16) * cdiv(w.k_in, 16) < ((int64_t)1 << 31) &&
-           (w.format == RQ_Q_ROWWISE_I8 || (w.group % 4 == 0 && w.k_in % w.group == 0));
+    if (!(aligned(w.codes, 4) && aligned(dy, dyt == RQ_F16 ? 8 : 16) && w.k_in % 4 == 0 && w.n_out % 4 == 0 &&
+          w.k_in * 64 < lim && w.n_out * 128 < lim &&
+          (w.format == RQ_Q_ROWWISE_I8 || (w.group % 4 == 0 && w.k_in % w.group == 0))))
+        return false;
+    const ChainTiles t = chain_tiles(m, w.k_in, num_cus);
+    return grid_ok(t.rows * t.cols, TH);
 }
 
 template <int FMT, bool DYF16>
@@ -333,7 +336,7 @@ int launch_chain(const rq_qweight &w, const void *dyv, void *dx, bool dxf16, int
 int launch_qmatmul_dx(const rq_qweight &w, const void *dy, rq_dtype dyt, void *dx, rq_dtype dxt, int64_t m,
                       int num_cus, hipStream_t s) {
     const bool dyf16 = dyt == RQ_F16, dxf16 = dxt == RQ_F16;
-    if (dx_chain_ok(w, dy, dyt, m)) {
+    if (dx_chain_ok(w, dy, dyt, m, num_cus)) {
         if (w.format == RQ_Q_ROWWISE_I8)
             return dyf16 ? launch_chain<RQ_Q_ROWWISE_I8, _Float16>(w, dy, dx, dxf16, m, num_cus, s)
                          : launch_chain<RQ_Q_ROWWISE_I8, float>(w, dy, dx, dxf16, m, num_cus, s);
@@ -620,3 +623,16 @@ int rq_qmatmul_dx_mfma(rq_ctx *ctx, const rq_qweight *w, const void *table, cons
 }
 
 }  // extern "C"
+
+// For the tests, no part of the C ABI: the tile (bm * 1000 + bn) of the
+// matrix-core kernel that serves an input gradient in f32 with aligned
+// operands, 0 for the VALU kernel.  Host arithmetic.
+extern "C" int rusty_dx_kernel(int fmt, int group, int64_t m, int64_t n_out, int64_t k_in, int num_cus) {
+    using namespace rq;
+    rq_qweight w{};
+    w.format = fmt;
+    w.group = group;
+    w.n_out = n_out;
+    w.k_in = k_in;
+    return dx_chain_ok(w, nullptr, RQ_F32, m, num_cus) ? chain_tile_id(chain_tiles(m, k_in, num_cus)) : 0;
+}

@@ -58,6 +58,9 @@ inline bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// HIP launches fewer than 2^32 threads along a grid dimension.
+inline bool grid_ok(int64_t blocks, int64_t threads) { return blocks * threads < ((int64_t)1 << 32); }
+
 // Launchers implemented in the kernel translation units.  Arguments are
 // validated by the C-ABI layer before these are called.
 int launch_dequantize(const uint32_t *in, size_t n_words, float *out, size_t n_out, hipStream_t s);

@@ -1061,6 +1061,11 @@ double tile_cost(int id, int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus)
     return us * (1.0 - 0.35 * (1.0 - fill)) * (id == T64x128 ? 1.08 : 1.0);
 }
 
+// Whether a grid of tile `id` can be launched (512 threads a block at most).
+bool tile_launches(int id, int64_t m, int64_t N) {
+    return grid_ok(cdiv(m, kTile[id].bm) * cdiv(N, kTile[id].bn), 512);
+}
+
 // The largest tile whose grid still has >= 2/3 as many tiles as the device has
 // CUs, unless the fitted times say that another is at least 5 % faster: a
 // round of tiles that is nearly empty costs as much as a full one.  128x256
@@ -1079,6 +1084,7 @@ int choose_tile(int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus) {
     int best = pick;
     double us = tile_cost(pick, fmt, m, N, nk, cus) * 0.95;
     for (int id = 0; id < kTiles; ++id) {
+        if (!tile_launches(id, m, N)) continue;
         const double c = tile_cost(id, fmt, m, N, nk, cus);
         if (c < us) {
             best = id;
@@ -1115,7 +1121,7 @@ int choose_pair_tile(int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus) {
     int best = pick;
     double us = pick < 0 ? (two + 3.0) * 0.9 : tile_cost(pick, fmt, m, N, nk, cus) * 0.95;
     for (int id : {T128x256, T192x128, T128x128, T64x128}) {
-        if (!pair_fits(id, I)) continue;
+        if (!pair_fits(id, I) || !tile_launches(id, m, N)) continue;
         const double c = tile_cost(id, fmt, m, N, nk, cus);
         if (c < us) {
             best = id;

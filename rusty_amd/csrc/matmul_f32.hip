@@ -456,10 +456,11 @@ int launch_chain(const void *a, const float *b, float *out, int64_t m, int64_t k
 
 // Offsets within a panel stay below 2^29 elements (ChainSpan): rows of up to
 // 4 M elements along k, 8 M along the outputs.
-bool mfma_fits(int v, int64_t m, int64_t k, int64_t n) {
+bool mfma_fits(int v, int64_t m, int64_t k, int64_t n, int num_cus) {
     const int64_t lim = (int64_t)1 << 29;
-    return (v == MM_ATB ? m * 64 < lim : k * 128 < lim) && (v == MM_ABT ? k * 128 < lim : n * 64 < lim) &&
-           cdiv(m, 16) * cdiv(n, 16) < ((int64_t)1 << 31);
+    if (!((v == MM_ATB ? m * 64 < lim : k * 128 < lim) && (v == MM_ABT ? k * 128 < lim : n * 64 < lim))) return false;
+    const ChainTiles t = chain_tiles(m, n, num_cus);
+    return grid_ok(t.rows * t.cols, MTH);
 }
 // Which kernel serves a product, measured on MI355X (us, VALU kernels ->
 // matrix cores, AB / ABT / ATB unless stated):
@@ -479,7 +480,7 @@ bool mfma_fits(int v, int64_t m, int64_t k, int64_t n) {
 //    292 -> 28, 512x4096x16 27.3 / 26.1 / 28.0 -> 24.7 / 24.7 / 27.0).
 enum Route { ROUTE_TILED, ROUTE_CHAIN, ROUTE_RING, ROUTE_MFMA };
 template <typename TA>
-Route route(int v, const TA *a, const float *b, int64_t m, int64_t k, int64_t n) {
+Route route(int v, const TA *a, const float *b, int64_t m, int64_t k, int64_t n, int num_cus) {
     if (k <= 16 || (k <= 48 && m * n > ((int64_t)1 << 21))) return ROUTE_TILED;
     const bool chain = k > 64 && chain_fits(m, k, n);
     if constexpr (std::is_same_v<TA, float>)
@@ -487,7 +488,7 @@ Route route(int v, const TA *a, const float *b, int64_t m, int64_t k, int64_t n)
     const int64_t tiles = cdiv(m, 16) * cdiv(n, 16);
     if (chain && k > 256 && tiles <= 1)
         return ROUTE_CHAIN;
-    return mfma_fits(v, m, k, n) ? ROUTE_MFMA : ROUTE_TILED;
+    return mfma_fits(v, m, k, n, num_cus) ? ROUTE_MFMA : ROUTE_TILED;
 }
 
 }  // namespace
@@ -495,7 +496,7 @@ Route route(int v, const TA *a, const float *b, int64_t m, int64_t k, int64_t n)
 int launch_matmul_f32(int variant, const float *a, const float *b, float *out, int64_t m, int64_t k, int64_t n,
                       int num_cus, hipStream_t s) {
     if (m == 0 || n == 0) return RQ_OK;
-    const Route r = route(variant, a, b, m, k, n);
+    const Route r = route(variant, a, b, m, k, n, num_cus);
     if (r == ROUTE_MFMA) {
         switch (variant) {
         case MM_AB: return launch_mfma_ab(a, b, out, m, k, n, num_cus, s);
@@ -534,7 +535,7 @@ int launch_matmul_f32(int variant, const float *a, const float *b, float *out, i
 int launch_matmul_f32_ah(const _Float16 *a, const float *b, float *out, int64_t m, int64_t k, int64_t n, int num_cus,
                          hipStream_t s) {
     if (m == 0 || n == 0) return RQ_OK;
-    switch (route(MM_AB, a, b, m, k, n)) {
+    switch (route(MM_AB, a, b, m, k, n, num_cus)) {
     case ROUTE_MFMA: return launch_mfma_ab_f16(a, b, out, m, k, n, num_cus, s);
     case ROUTE_CHAIN: return launch_chain<MM_AB, true>(a, b, out, m, k, n, s);
     default: return RQ_ERR_UNSUPPORTED;
@@ -542,3 +543,13 @@ int launch_matmul_f32_ah(const _Float16 *a, const float *b, float *out, int64_t 
 }
 
 }  // namespace rq
+
+// For the tests, no part of the C ABI: the kernel that serves a product with
+// 16-byte aligned f32 operands.  0 tiled, 1 register-staged chains, 2 ring
+// chains, the tile (bm * 1000 + bn) on the matrix cores.  Host arithmetic.
+extern "C" int rusty_matmul_kernel(int variant, int64_t m, int64_t k, int64_t n, int num_cus) {
+    using namespace rq;
+    const float *aligned16 = reinterpret_cast<const float *>(uintptr_t(64));
+    const Route r = route(variant, aligned16, aligned16, m, k, n, num_cus);
+    return r == ROUTE_MFMA ? chain_tile_id(chain_tiles(m, n, num_cus)) : (int)r;
+}

@@ -476,6 +476,18 @@ inline ChainTiles chain_tiles(int64_t m, int64_t n, int num_cus) {
     return best;
 }
 
+// bm * 1000 + bn of a choice (for the tests).
+inline int chain_tile_id(const ChainTiles &t) {
+    switch (t.shape) {
+    case CHAIN_128: return 128128;
+    case CHAIN_64: return 64064;
+    case CHAIN_32: return 32032;
+    case CHAIN_16x64: return 16064;
+    case CHAIN_64x16: return 64016;
+    }
+    return -1;
+}
+
 // Tile of block `id` among rows x cols tiles: the blocks an XCD runs (ids
 // round-robin over 8) take consecutive tiles, in groups of 8 tile rows walked
 // column by column, so that they share operand panels in that XCD's L2.

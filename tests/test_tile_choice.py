@@ -22,6 +22,42 @@ def gemm_tile(fmt, m, n_out, k_in, pair=False):
     return None if t < 0 else divmod(t, 1000)
 
 
+def matmul_kernel(variant, m, k, n):
+    """0 tiled, 1 register-staged chains, 2 ring chains, else the matrix-core tile (rows, columns)."""
+    i32, i64 = ctypes.c_int, ctypes.c_int64
+    t = _fn("rusty_matmul_kernel", i32, i64, i64, i64, i32)(variant, m, k, n, CUS)
+    return t if t < 1000 else divmod(t, 1000)
+
+
+def dx_kernel(fmt, group, m, n_out, k_in):
+    """0 for the VALU kernel, else the matrix-core tile (rows, columns)."""
+    i32, i64 = ctypes.c_int, ctypes.c_int64
+    t = _fn("rusty_dx_kernel", i32, i32, i64, i64, i64, i32)(fmt, group, m, n_out, k_in, CUS)
+    return t if t < 1000 else divmod(t, 1000)
+
+
+def _threads(t, m, n, per_block):
+    return -(-m // t[0]) * -(-n // t[1]) * per_block
+
+
+@pytest.mark.parametrize("big", [1 << 27, (1 << 29) - 8, 1 << 29, (1 << 29) + 40, 1 << 30])
+@pytest.mark.parametrize("small", [1, 8, 17, 32, 64, 100])
+def test_grids_stay_below_the_launch_limit(big, small):
+    """A launch has fewer than 2^32 threads along x: no rule moves a product
+    whose larger tiles fit that to smaller ones that do not."""
+    for m, n in ((small, big), (big, small)):
+        for variant in range(3):
+            for k in (56, 260):
+                t = matmul_kernel(variant, m, k, n)
+                assert isinstance(t, int) or _threads(t, m, n, 256) < 1 << 32, (variant, m, k, n, t)
+        for fmt, group in ((0, 0), (1, 4)):
+            t = dx_kernel(fmt, group, m, 64, n & ~3)
+            assert isinstance(t, int) or _threads(t, m, n & ~3, 256) < 1 << 32, (fmt, m, n, t)
+            for width in (64, 128, 200, 256):
+                t = gemm_tile(fmt, min(big, (1 << 29) + 40), width, 64)
+                assert _threads(t, min(big, (1 << 29) + 40), width, 512 if t[1] >= 128 else 256) < 1 << 32, (width, t)
+
+
 @pytest.mark.parametrize("fmt", [0, 1])
 def test_pair_tile_rows_stay_below_the_mask_offset(fmt):
     """The fused gate/up copy-out masks pieces with byte offset 2^31: no tile's
