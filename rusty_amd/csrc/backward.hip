@@ -293,7 +293,7 @@ bool dx_chain_ok(const rq_qweight &w, const void *dy, rq_dtype dyt, int64_t m, i
           w.k_in * 64 < lim && w.n_out * 128 < lim &&
           (w.format == RQ_Q_ROWWISE_I8 || (w.group % 4 == 0 && w.k_in % w.group == 0))))
         return false;
-    const ChainTiles t = chain_tiles(m, w.k_in, num_cus);
+    const ChainTiles t = chain_tiles(m, w.k_in, w.n_out, num_cus);
     return grid_ok(t.rows * t.cols, TH);
 }
 
@@ -313,7 +313,7 @@ int launch_fmt(const rq_qweight &w, const void *dy, void *dx, bool dxf16, int64_
 
 template <int FMT, typename TY>
 int launch_chain(const rq_qweight &w, const void *dyv, void *dx, bool dxf16, int64_t m, int num_cus, hipStream_t s) {
-    const ChainTiles t = chain_tiles(m, w.k_in, num_cus);
+    const ChainTiles t = chain_tiles(m, w.k_in, w.n_out, num_cus);
     const dim3 grid((unsigned)(t.rows * t.cols));
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(TH), 0, s, static_cast<const uint8_t *>(w.codes), w.scales, w.biases,
@@ -634,5 +634,5 @@ extern "C" int rusty_dx_kernel(int fmt, int group, int64_t m, int64_t n_out, int
     w.group = group;
     w.n_out = n_out;
     w.k_in = k_in;
-    return dx_chain_ok(w, nullptr, RQ_F32, m, num_cus) ? chain_tile_id(chain_tiles(m, k_in, num_cus)) : 0;
+    return dx_chain_ok(w, nullptr, RQ_F32, m, num_cus) ? chain_tile_id(chain_tiles(m, k_in, n_out, num_cus)) : 0;
 }

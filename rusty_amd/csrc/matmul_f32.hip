@@ -459,7 +459,7 @@ int launch_chain(const void *a, const float *b, float *out, int64_t m, int64_t k
 bool mfma_fits(int v, int64_t m, int64_t k, int64_t n, int num_cus) {
     const int64_t lim = (int64_t)1 << 29;
     if (!((v == MM_ATB ? m * 64 < lim : k * 128 < lim) && (v == MM_ABT ? k * 128 < lim : n * 64 < lim))) return false;
-    const ChainTiles t = chain_tiles(m, n, num_cus);
+    const ChainTiles t = chain_tiles(m, n, k, num_cus);
     return grid_ok(t.rows * t.cols, MTH);
 }
 // Which kernel serves a product, measured on MI355X (us, VALU kernels ->
@@ -551,5 +551,5 @@ extern "C" int rusty_matmul_kernel(int variant, int64_t m, int64_t k, int64_t n,
     using namespace rq;
     const float *aligned16 = reinterpret_cast<const float *>(uintptr_t(64));
     const Route r = route(variant, aligned16, aligned16, m, k, n, num_cus);
-    return r == ROUTE_MFMA ? chain_tile_id(chain_tiles(m, n, num_cus)) : (int)r;
+    return r == ROUTE_MFMA ? chain_tile_id(chain_tiles(m, n, k, num_cus)) : (int)r;
 }

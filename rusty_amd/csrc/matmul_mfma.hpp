@@ -68,7 +68,7 @@ __global__ __launch_bounds__(MTH, MINB) void k_matmul_mfma(const TA *__restrict_
 template <int V, typename TA, bool VA, bool VB>
 int launch_mfma_vec(const TA *a, const float *b, float *out, int64_t m, int64_t k, int64_t n, int num_cus,
                     hipStream_t s) {
-    const ChainTiles t = chain_tiles(m, n, num_cus);
+    const ChainTiles t = chain_tiles(m, n, k, num_cus);
     const dim3 grid((unsigned)(t.rows * t.cols));
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(MTH), 0, s, a, b, out, m, k, n, (uint32_t)t.rows, (uint32_t)t.cols);

@@ -440,34 +440,43 @@ struct ChainTile {
 };
 
 // ---- tiles -------------------------------------------------------------------------
-// Tile shapes and their time per k-step and round of one block per CU, measured
-// on MI355X at k = 4096, operands in cache (ns; the matrix instructions alone
-// need 53 / 13.2 / 3.3):
-//   128x128, 32x32x2, KC 32   65 (4 blocks per CU, 4096^3: 1075 us, 128 TFLOP/s)
-//   64x64,   32x32x2, KC 32   16.7 (2 per CU, 512x4096x4096: 134-137 us)
-//   32x32, 16x64, 64x16, 16x16x4, KC 64   6.1 (1 per CU), 5.3 per further round
+// Tile shapes and the time of a round of one block per CU on MI355X, operands
+// in cache: ns per k-step (the matrix instructions alone need 53 / 13.2 / 3.3)
+// and, for its first loads and its outputs' write, us per round:
+//   128x128, 32x32x2, KC 32   60, 7.5 (4 blocks per CU, 4096^3: 978-986 us, 140 TFLOP/s)
+//   64x64,   32x32x2, KC 32   16.7, 1.3 (2 per CU, 512x4096x4096: 134-137 us)
+//   32x32, 16x64, 64x16, 16x16x4, KC 64   6.1 (1 per CU), 5.3 per further round; 0.5
 //            (512x4096x16 24.5 us, 16x4096x4096 25 us)
 // The one with the least total is taken: large tiles waste what a ragged edge
 // or an unfilled round leaves idle, small ones read each operand more often.
+// A 128x128 tile writes its 64 KiB at the end, with no second block on its CU
+// to multiply meanwhile, so short reductions take 64x64 ones (us, 128x128 ->
+// 64x64: 2048x4096 outputs of k = 64 21.4 -> 17.7, 128 28.8 -> 26.0, 256 43.3 ->
+// 40.6; at 2048x2048 of k = 512 38.5 against 41.1, so 128x128 stays), and 64x64
+// rather than 32x32 (700x3000 of k = 64 9.7 -> 7.6, a gradient of k = 20 11.4 -> 7.3).  Over
+// 177 products and gradients of k = 20 .. 2048 the choice is within 0.5 % of
+// the best tile on average, 6 % without the time per round, and never more
+// than 0.4 % slower than without it.
 enum ChainShape { CHAIN_128, CHAIN_64, CHAIN_32, CHAIN_16x64, CHAIN_64x16 };
 struct ChainTiles {
     ChainShape shape;
     int64_t rows, cols;  // tiles along m and n
 };
-inline ChainTiles chain_tiles(int64_t m, int64_t n, int num_cus) {
+inline ChainTiles chain_tiles(int64_t m, int64_t n, int64_t k, int num_cus) {
     struct Cand {
         ChainShape shape;
         int bm, bn;
-        double first, more;
+        double first, more, round;
     };
-    static constexpr Cand cands[] = {{CHAIN_128, 128, 128, 65, 65},      {CHAIN_64, 64, 64, 16.7, 16.7},
-                                     {CHAIN_32, 32, 32, 6.1, 5.3},       {CHAIN_16x64, 16, 64, 6.2, 5.4},
-                                     {CHAIN_64x16, 64, 16, 6.2, 5.4}};
+    static constexpr Cand cands[] = {{CHAIN_128, 128, 128, 60, 60, 7.5},  {CHAIN_64, 64, 64, 16.7, 16.7, 1.3},
+                                     {CHAIN_32, 32, 32, 6.1, 5.3, 0.5},   {CHAIN_16x64, 16, 64, 6.2, 5.4, 0.5},
+                                     {CHAIN_64x16, 64, 16, 6.2, 5.4, 0.5}};
     ChainTiles best{};
     double cost = 0;
     for (const Cand &c : cands) {
         const int64_t r = cdiv(m, c.bm), q = cdiv(n, c.bn);
-        const double t = c.first + c.more * (double)(cdiv(r * q, num_cus) - 1);
+        const double rounds = (double)cdiv(r * q, num_cus);
+        const double t = (c.first + c.more * (rounds - 1)) * (double)k * 1e-3 + c.round * rounds;
         if (&c == cands || t < cost) {
             best = {c.shape, r, q};
             cost = t;

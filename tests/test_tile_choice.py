@@ -73,3 +73,15 @@ def test_pair_tile_rows_stay_below_the_mask_offset(fmt):
                     served += 1
                     assert t[0] * inter * 2 < 1 << 31, (m, inter, k, t)
     assert served > 50  # widths below 128-row tiles' limit are still one launch
+
+
+def test_short_reductions_take_smaller_tiles():
+    """A round of 128x128 tiles has a fixed cost (its outputs' write) that a
+    short reduction does not hide: 64x64 there, 128x128 for long ones."""
+    for k in (64, 128, 256):
+        assert all(matmul_kernel(v, 2048, k, 4096) == (64, 64) for v in range(3))
+        assert dx_kernel(0, 0, 2048, k, 4096) == dx_kernel(1, 64, 2048, k, 4096) == (64, 64)
+    for k in (64, 128, 256):
+        assert matmul_kernel(0, 700, k, 3000) == (64, 64)
+    assert matmul_kernel(0, 2048, 512, 2048) == matmul_kernel(0, 4096, 4096, 4096) == (128, 128)
+    assert matmul_kernel(0, 512, 4096, 16) == (32, 32)
