@@ -20,7 +20,7 @@
 // k_dx_chain runs on the f32 matrix cores (mfma_chain.hpp) and serves every
 // call whose codes come in words (dx_chain_ok); k_qmatmul_dx, on the VALU,
 // the rest (k_in or n_out not a multiple of 4, unaligned operands, groups that
-// do not divide k_in).  Bound by the matrix instructions, which share the SIMD
+// do not divide k_in) and short reductions into many outputs (dx_short).  Bound by the matrix instructions, which share the SIMD
 // with the dequantization (3-4 VALU instructions per element of a tile, for
 // 64 or 128 rows' products): us, VALU -> matrix cores, 512x4096x4096 affine 518 -> 140,
 // per-row 372 -> 139; 2048x4096x4096 affine 1616 -> 587; 16 rows x 11008x4096
@@ -297,6 +297,21 @@ bool dx_chain_ok(const rq_qweight &w, const void *dy, rq_dtype dyt, int64_t m, i
     return grid_ok(t.rows * t.cols, TH);
 }
 
+// A gradient of one step of the VALU kernel (32 of n_out) is its output's
+// write and a tile's fixed cost, of which that kernel, with more blocks in
+// flight, has less: it serves such calls from the output counts below on (f32
+// dY and dX, us, matrix cores -> VALU kernel, per-row, then affine: 512x4096
+// outputs, n_out 4 6.8 -> 6.2, 7.0 -> 7.3; 28 6.5 -> 6.1, 7.0 -> 7.6; 1024x4096,
+// 28 10.9 -> 9.6, 11.5 -> 11.0; 4096x4096, 4 29.0 -> 22.4, 30.8 -> 24.8; 28 29.0 ->
+// 24.0, 30.7 -> 28.0; 32 27.6 -> 25.9, 28.7 -> 31.1, at k_in % 8 = 4 17.3 -> 18.9;
+// from 36 on the matrix cores: 2048x4096 20.9 against 23.4).
+bool dx_short(const rq_qweight &w, int64_t m) {
+    if (cdiv(m, BM) > 65535) return false;  // the VALU kernel's grid
+    const bool rowwise = w.format == RQ_Q_ROWWISE_I8;
+    auto from = [&](int log2) { return m * w.k_in >= ((int64_t)1 << log2); };
+    return w.n_out <= (rowwise && from(23) && w.k_in % 8 == 0 ? 32 : from(rowwise ? 21 : 22) ? 28 : 0);
+}
+
 template <int FMT, bool DYF16>
 int launch_fmt(const rq_qweight &w, const void *dy, void *dx, bool dxf16, int64_t m, dim3 grid, hipStream_t s) {
     const uint8_t *codes = static_cast<const uint8_t *>(w.codes);
@@ -336,7 +351,7 @@ int launch_chain(const rq_qweight &w, const void *dyv, void *dx, bool dxf16, int
 int launch_qmatmul_dx(const rq_qweight &w, const void *dy, rq_dtype dyt, void *dx, rq_dtype dxt, int64_t m,
                       int num_cus, hipStream_t s) {
     const bool dyf16 = dyt == RQ_F16, dxf16 = dxt == RQ_F16;
-    if (dx_chain_ok(w, dy, dyt, m, num_cus)) {
+    if (dx_chain_ok(w, dy, dyt, m, num_cus) && !dx_short(w, m)) {
         if (w.format == RQ_Q_ROWWISE_I8)
             return dyf16 ? launch_chain<RQ_Q_ROWWISE_I8, _Float16>(w, dy, dx, dxf16, m, num_cus, s)
                          : launch_chain<RQ_Q_ROWWISE_I8, float>(w, dy, dx, dxf16, m, num_cus, s);
@@ -634,5 +649,6 @@ extern "C" int rusty_dx_kernel(int fmt, int group, int64_t m, int64_t n_out, int
     w.group = group;
     w.n_out = n_out;
     w.k_in = k_in;
-    return dx_chain_ok(w, nullptr, RQ_F32, m, num_cus) ? chain_tile_id(chain_tiles(m, k_in, n_out, num_cus)) : 0;
+    if (!dx_chain_ok(w, nullptr, RQ_F32, m, num_cus) || dx_short(w, m)) return 0;
+    return chain_tile_id(chain_tiles(m, k_in, n_out, num_cus));
 }

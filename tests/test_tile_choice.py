@@ -85,3 +85,18 @@ def test_short_reductions_take_smaller_tiles():
         assert matmul_kernel(0, 700, k, 3000) == (64, 64)
     assert matmul_kernel(0, 2048, 512, 2048) == matmul_kernel(0, 4096, 4096, 4096) == (128, 128)
     assert matmul_kernel(0, 512, 4096, 16) == (32, 32)
+
+
+@pytest.mark.parametrize("fmt,group,rows", [(0, 0, 512), (1, 64, 1024)])
+def test_short_input_gradients_of_many_outputs(fmt, group, rows):
+    """One step of the VALU kernel into many outputs is its; anything longer or
+    smaller, and more rows than its grid takes, the matrix cores'."""
+    for m in (rows, 2 * rows, 8192):
+        for n_out in (4, 16, 28):
+            assert dx_kernel(fmt, group, m, n_out, 4096) == 0
+        assert dx_kernel(fmt, group, m, 36, 4096) != 0
+    assert dx_kernel(fmt, group, rows - 64, 28, 4096) != 0
+    assert (dx_kernel(fmt, group, 2048, 32, 4096) == 0) == (fmt == 0)
+    assert dx_kernel(fmt, group and 4, 2048, 32, 4100) != 0
+    assert dx_kernel(fmt, group, 512, 256, 4096) != 0
+    assert dx_kernel(fmt, group, 65535 * 64 + 1, 16, 256) != 0
