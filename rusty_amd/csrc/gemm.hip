@@ -781,7 +781,14 @@ __global__ __launch_bounds__(64 * NW) void k_gemm_rowwise(const uint8_t *__restr
                 v = __builtin_bit_cast(uint4, hv);
             }
             const uint32_t off = col_ok ? (uint32_t)row * (uint32_t)NL * OE + (uint32_t)c * 16u : kOOB;
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, off, 0, 2);
+            // non-temporal, except an h of a width that the down product's GEMM does not
+            // take (k_in % 64): the generic kernel reads it many times over (MLP of 137 x
+            // (5288, 1408) 1219 us with h streamed past the caches, 1084 without; streamed h
+            // read once by the GEMM is 2 % faster or up to 7 % slower by shape)
+            if (PAIR && NL % 64 != 0)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, off, 0, 0);
+            else
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), ry, off, 0, 2);
         }
     };
     if constexpr (ROPE) {
