@@ -124,10 +124,15 @@ __device__ __forceinline__ half8 u8x8_affine(uint2 w, float s, float c) {
 }
 
 // Tile order: consecutive blocks go round-robin to the 8 XCDs, so block b
-// runs on XCD b % 8; it takes position L = its XCD's first tile + b / 8 of
-// a group-M order (XCDs below tiles % 8 hold one tile more) (GM m-tiles per group, n-tiles across, m fastest within a
-// group).  The 32 concurrent tiles of one XCD then cover GM token panels x
-// 32/GM feature panels, so both X and W panels are reused in that XCD's L2.
+// runs on XCD b % 8; it takes position L = its XCD's first tile + b / 8 (XCDs
+// below tiles % 8 hold one tile more) of a group-M order (GM m-tiles per
+// group, n-tiles across, m fastest within a group).  The 32 concurrent tiles
+// of one XCD then cover GM token panels x 32/GM feature panels, so both X and
+// W panels are reused in that XCD's L2.  On grids that are no multiple of 8 this is
+// a gain on average, not on each: against L = b there, over 153 random products, 1.014x
+// (0.91-1.16x; weights of over 8 MiB 1.03x, none below 0.98: 177x6296x3392 22.7 ->
+// 19.6 us, 777x11008x4096 affine 109 -> 105; tall ones lose: 1293x896x2624 14.4 ->
+// 15.8).  L = b for weights up to 8 MiB, for tall grids or for splits of K lost as much elsewhere.
 __device__ __forceinline__ void tile_of(int b, int tiles_m, int tiles_n, int gm, int &tm, int &tn) {
     const int tiles = tiles_m * tiles_n;  // b < tiles
     const int x = b % 8, L = x * (tiles / 8) + min(x, tiles % 8) + b / 8;
@@ -1082,17 +1087,27 @@ bool tile_launches(int id, int64_t m, int64_t N) {
 // the rounds between (us, before -> after: 2048x2560x2048 35.8 -> 25.3,
 // 1536x4096x4096 57.6 -> 49.3, 777x11008x4096 affine 117.5 -> 101.3; SwiGLU
 // pairs, with the down product, 300x5632x2048 59.1 -> 43.6, 128x5632x2048
-// 40.0 -> 25.9, 1536x5632x2048 148.5 -> 133.9; over 140 random shapes 0.95-1.74x).
-// 64x256 was never the best.  A 64x64 grid that would split K (launch_tiled) stays.
+// 40.0 -> 25.9, 1536x5632x2048 148.5 -> 133.9; over 160 random products whose
+// tile changed 0.94-2.1x, 1.27x on average).  64x256 was never the best.  A
+// 64x64 grid that would split K (launch_tiled) stays, on a caller's own
+// stream too, where there is no workspace to split with: as without the fit.
 int choose_tile(int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus) {
     auto fills = [&](int id) { return tile_fills(m, N, cus, kTile[id].bm, kTile[id].bn); };
     const int pick = fills(T128x256) ? T128x256 : fills(T128x128) ? T128x128 : fills(T128x64) ? T128x64 : T64x64;
     if (pick == T64x64 && 4 * cdiv(m, 64) * cdiv(N, 64) <= 3 * cus) return pick;  // split K
+    // One round of 128x256 tiles over a short K, which the fit (K = 1024 and 4096)
+    // does not cover: its output's write bounds it (554x10904x320 13.2 us,
+    // 64x128 15.0; 1179x4672x384 16.6, 64x64 17.0; 1106x5816x256 13.7, 64x128 13.3).
+    if (pick == T128x256 && nk < 8 && cdiv(m, 128) * cdiv(N, 256) <= cus) return pick;
+    // Three 64x64 tiles of per-row codes on a CU take up to 1.2x what the fit, its
+    // operands in cache, has for them: 8 % more before another tile gives way to
+    // them (1066x2720x1152 128x128 13.1 us, 64x64 13.6).
+    const bool crowded = fmt == 0 && cdiv(m, 64) * cdiv(N, 64) > 2 * cus;
     int best = pick;
     double us = tile_cost(pick, fmt, m, N, nk, cus) * 0.95;
     for (int id = 0; id < kTiles; ++id) {
         if (!tile_launches(id, m, N)) continue;
-        const double c = tile_cost(id, fmt, m, N, nk, cus);
+        const double c = tile_cost(id, fmt, m, N, nk, cus) * (id == T64x64 && crowded ? 1.08 : 1.0);
         if (c < us) {
             best = id;
             us = c;
@@ -1108,7 +1123,9 @@ bool pair_fits(int id, int64_t I) { return kTile[id].bm * I * 2 < (int64_t)kOOB;
 
 // Gate and up as one grid (PAIR): the tiles of 128 columns and more, against
 // two products and the silu*mul pass over their results (about 3 us more
-// than the two): -1.
+// than the two): -1.  Two small products are priced with their split of K; on a
+// caller's own stream, which has no workspace for it, they take longer than
+// that, and one grid would be the faster way for some calls that run as two.
 int choose_pair_tile(int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus) {
     const int64_t I = N / 2;
     if (!pair_fits(T128x256, I)) return -1;
@@ -1212,7 +1229,12 @@ int launch_gemm_qkv_rope(const rq_qweight &w, const _Float16 *x, int64_t m, cons
     const float *sc = affine ? w.prep : w.scales;
     const int fmt = affine ? 1 : 0;
     // the 64-wide tiles against the best tile and a rotation pass over its f32
-    // rows (6 bytes per value at ~4.5 TB/s, 2 us of launch)
+    // rows (6 bytes per value at ~4.5 TB/s, 2 us of launch).  The prices carry
+    // past the three tiles per CU they were fitted to: over prompts of 64 .. 2048
+    // positions at 2560x2048 and 5120x4096 the choice costs 0.3 us a layer on
+    // average, 3 at most, against the best of the three (2048 positions at 2560x2048, five
+    // 64x64 tiles per CU: 945 us for 4 layers, 953 with a rotation pass, 988 on 128x64;
+    // 1280 at 5120x4096: 597 for 3 layers with the pass, 645, 677).
     const double a = tile_cost(T128x64, fmt, m, N, K / 64, cus), b = tile_cost(T64x64, fmt, m, N, K / 64, cus);
     const double pass = 2.0 + 6e-6 / 4.5 * (double)m * (double)N;
     if (std::min(a, b) > tile_cost(choose_tile(fmt, m, N, K / 64, cus), fmt, m, N, K / 64, cus) + pass)

@@ -100,3 +100,15 @@ def test_short_input_gradients_of_many_outputs(fmt, group, rows):
     assert dx_kernel(fmt, group and 4, 2048, 32, 4100) != 0
     assert dx_kernel(fmt, group, 512, 256, 4096) != 0
     assert dx_kernel(fmt, group, 65535 * 64 + 1, 16, 256) != 0
+
+
+def test_gemm_tile_outside_the_fitted_times():
+    """What the fitted times miss: one round of 128x256 tiles over a short K
+    stays, three 64x64 tiles per CU need a clear gain; measured the other way
+    round, both lost."""
+    for m, n, k in ((554, 10904, 320), (1179, 4672, 384), (922, 6579, 320)):
+        assert gemm_tile(0, m, n, k) == (128, 256)
+    assert gemm_tile(0, 1453, 6816, 384) == (64, 128)  # more than a round: 23.3 us on 128x256, 18.4
+    assert gemm_tile(0, 1066, 2720, 1152) == (128, 128)
+    assert gemm_tile(0, 157, 8448, 896) == (64, 64)  # 128x64 17.3 us, 64x64 8.5
+    assert gemm_tile(1, 390, 4992, 1408) == (64, 64)
