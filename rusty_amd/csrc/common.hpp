@@ -182,7 +182,7 @@ int launch_rope_scatter(const float *qkv, const float2 *rope, int p0, int n, int
 // Causal attention of the n queries at positions p0.. (p0 % 32 == 0) over
 // cache positions 0..p0+n-1; out fp16 [n][n_heads * hd].
 int launch_attn_prefill(const _Float16 *q, const _Float16 *kc, const _Float16 *vc, _Float16 *out, int p0, int n,
-                        int n_heads, int n_kv, int hd, int max_seq, hipStream_t s);
+                        int n_heads, int n_kv, int hd, int max_seq, int num_cus, hipStream_t s);
 
 // Y = X . deq(W)^T over every kernel family, picked by m, dtypes and shape;
 // the prefill GEMM may use ws (split-K partials, input preparation).

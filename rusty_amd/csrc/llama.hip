@@ -533,7 +533,7 @@ int prefill_chunk(rq_llama *md, int p0, int n, bool end, hipStream_t s) {
         }
         if (l == c.n_layers - 1) break;  // the last layer's rest: below, for the last position only
         if ((st = launch_attn_prefill(md->pq, kc, vc, md->patt, p0, n, c.n_heads, c.n_kv_heads, c.head_dim,
-                                      c.max_seq, s)))
+                                      c.max_seq, md->ctx->num_cus, s)))
             return st;
         if ((st = qmatmul_dispatch(md->ctx, L.o, md->patt, RQ_F16, md->py, RQ_F32, n, ws, s))) return st;
         if ((st = launch_add_rmsnorm_rows(md->px, md->py, L.mlp_norm, c.norm_eps, md->pxn, n, H, s))) return st;
@@ -551,7 +551,7 @@ int prefill_chunk(rq_llama *md, int p0, int n, bool end, hipStream_t s) {
         const int t0 = 32 * ((n - 1) / 32);  // first row of the last query tile
         if ((st = launch_attn_prefill(md->pq + t0 * qrow, md->kc + l * kv_layer, md->vc + l * kv_layer,
                                       md->patt + t0 * qrow, p0 + t0, n - t0, c.n_heads, c.n_kv_heads, c.head_dim,
-                                      c.max_seq, s)))
+                                      c.max_seq, md->ctx->num_cus, s)))
             return st;
         const size_t last = (size_t)(n - 1);
         if ((st = qmatmul_dispatch(md->ctx, L.o, md->patt + last * qrow, RQ_F16, md->py + last * H, RQ_F32, 1, ws, s)))

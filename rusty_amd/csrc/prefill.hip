@@ -572,14 +572,16 @@ int launch_rope_scatter(const float *qkv, const float2 *rope, int p0, int n, int
 }
 
 int launch_attn_prefill(const _Float16 *q, const _Float16 *kc, const _Float16 *vc, _Float16 *out, int p0, int n,
-                        int n_heads, int n_kv, int hd, int max_seq, hipStream_t s) {
+                        int n_heads, int n_kv, int hd, int max_seq, int num_cus, hipStream_t s) {
     if (p0 % 32 != 0 || n < 1 || (hd != 64 && hd != 128) || n_heads % n_kv != 0) return RQ_ERR_UNSUPPORTED;
-    // Blocks of 128 queries from three quarters of a 256-CU device on (us for
-    // three layers' attention and the rest of a 4-layer 1.1B-shape prompt, small
-    // blocks -> these: 768 positions 542 -> 529, 1024 628 -> 615, 2048 1047 ->
-    // 939, 4096 2388 -> 1942; 512, 128 blocks, 389 -> 397).
+    // Blocks of 128 queries where they cover three quarters of the CUs (256 CUs, us
+    // per layer, small blocks -> these, after 0 / 2048 / 6144 cached positions: 32 heads of 64,
+    // 768 positions (192 blocks) 20.1 -> 13.0, 61 -> 38, 148 -> 101, 2048 77 -> 32,
+    // 190 -> 72, 415 -> 153; 64 heads of 128, 257 positions (192 blocks, a third
+    // of them with one query) 23.7 -> 11.7, 130 -> 57, 341 -> 148; 32 heads of 64, 512
+    // positions (128 blocks), in a 4-layer prompt: 389 against 397).
     const int blocks = n_heads * ((n + 127) / 128);
-    if (blocks >= 192) {
+    if (4 * blocks >= 3 * num_cus) {
         if (hd == 64)
             hipLaunchKernelGGL((k_attn_prefill_rows<64>), dim3((unsigned)blocks), dim3(256), 0, s, q, kc, vc, out, p0,
                                n, n_heads, n_kv, max_seq);
