@@ -603,3 +603,17 @@ int launch_attn_prefill(const _Float16 *q, const _Float16 *kc, const _Float16 *v
 }
 
 }  // namespace rq
+
+// For the tests, no part of the C ABI: the prompt attention of a runner's layer
+// on the context's stream; q and out fp16 [n][n_heads][hd], kc and vc fp16
+// [n_kv][max_seq][hd], p0 a multiple of 32.
+extern "C" int rusty_attn_prefill(rq_ctx *ctx, const void *q, const void *kc, const void *vc, void *out, int p0, int n,
+                                  int n_heads, int n_kv, int hd, int max_seq) {
+    using namespace rq;
+    RQ_ENTER(ctx);
+    if (!q || !kc || !vc || !out || p0 < 0 || n < 1 || n_kv < 1 || p0 + n > max_seq)
+        return fail(RQ_ERR_INVALID_ARGUMENT, "attention arguments");
+    return launch_attn_prefill(static_cast<const _Float16 *>(q), static_cast<const _Float16 *>(kc),
+                               static_cast<const _Float16 *>(vc), static_cast<_Float16 *>(out), p0, n, n_heads, n_kv,
+                               hd, max_seq, ctx->num_cus, ctx->stream);
+}

@@ -12,11 +12,13 @@ TOL = 1e-2 for the small configs, 2e-2 for the 22-layer 1.1B shape: the
 device rounds GEMV inputs, the attention output and the KV cache to fp16
 (relative 2^-11 each), and the difference grows with depth.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
 from oracle import llama as ol
-from rusty_amd import RqError
+from rusty_amd import DType, RqError, UnifiedTensor, _lib
 from mlx_files import write_mlx_llama
 from rusty_amd.llama import LLAMA_1B, LlamaConfig, LlamaRunner, load_mlx, synth_weights
 
@@ -324,15 +326,68 @@ def _check_steps_pick(dec, ties):
             assert np.count_nonzero(lg == lg.max()) >= 2, (i, lg.max())
 
 
+def _attention_rows(q, k, v, p0, rows):
+    """float64 causal attention of query rows `rows`: outputs, and a bound on
+    what fp16 weights and outputs may differ by.
+
+    P is rounded to fp16 (2^-11 relative; below 2^-14 to a multiple of 2^-24,
+    with P's largest value at least 1), the output once more; scores, exponents
+    and sums are f32 (2^-13 relative on P covers exponents up to 2^9)."""
+    n_heads, hd, n_kv = q.shape[1], q.shape[2], k.shape[0]
+    out = np.zeros((len(rows), n_heads, hd))
+    bound = np.zeros_like(out)
+    for h in range(n_heads):
+        g = h // (n_heads // n_kv)
+        kg, vg = k[g].astype(np.float64), v[g].astype(np.float64)
+        s = q[rows, h].astype(np.float64) @ kg.T / np.sqrt(hd)
+        s[np.arange(len(kg))[None, :] > p0 + np.asarray(rows)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        norm = p.sum(1, keepdims=True)
+        out[:, h] = p @ vg / norm
+        keys = (p0 + np.asarray(rows) + 1)[:, None]
+        bound[:, h] = 2.0**-11 * np.abs(out[:, h]) + 2.0**-24 + (
+            (2.0**-11 + 2.0**-13) * (p @ np.abs(vg)) + keys * 2.0**-25 * np.abs(vg).max()) / norm
+    return out, bound
+
+
+# Both kernels (128-query blocks where they cover 192 of 256 CUs), both head sizes: partial last
+# blocks, tiles of 64 keys that start at p0 % 64 == 0 and 32, cached positions before the chunk.
+@pytest.mark.parametrize("n_heads,n_kv,hd,p0,n", [(16, 4, 64, 0, 1555), (16, 2, 64, 1568, 1421), (48, 6, 64, 2016, 417),
+                                                  (16, 16, 128, 96, 1601), (64, 8, 128, 2080, 257), (48, 48, 64, 32, 512),
+                                                  (4, 2, 64, 32, 77), (8, 8, 128, 96, 130), (32, 4, 64, 64, 640)])
+@pytest.mark.parametrize("sharp", [1.0, 6.0])
+def test_attention_rows(ctx, n_heads, n_kv, hd, p0, n, sharp):
+    """The prompt attention of one layer, every row of every head against
+    float64.  `sharp` spreads the scores over many powers of two, so that the
+    running maximum rises in steps past the rescaling threshold.  What lies
+    behind the chunk in the caches is NaN and must not be read."""
+    f = _lib.lib().rusty_attn_prefill
+    f.argtypes, f.restype = [ctypes.c_void_p] * 5 + [ctypes.c_int] * 6, ctypes.c_int
+    g = np.random.default_rng(n)
+    kv, seq = p0 + n, -(-(p0 + n + 70) // 32) * 32
+    q = (g.standard_normal((n, n_heads, hd), dtype=np.float32) * sharp).astype(np.float16)
+    k, v = (np.full((n_kv, seq, hd), np.nan, np.float16) for _ in range(2))
+    k[:, :kv] = g.standard_normal((n_kv, kv, hd), dtype=np.float32)
+    v[:, :kv] = g.standard_normal((n_kv, kv, hd), dtype=np.float32)
+    Q, K, V = (UnifiedTensor.new(ctx, a, dtype=DType.FP16) for a in (q, k, v))
+    out = UnifiedTensor.new(ctx, np.full((n, n_heads, hd), np.nan, np.float16), dtype=DType.FP16)
+    assert f(ctx.handle, Q.ptr, K.ptr, V.ptr, out.ptr, p0, n, n_heads, n_kv, hd, seq) == 0
+    got = out.to_vec().reshape(n, n_heads, hd).astype(np.float64)
+    for r0 in range(0, n, 256):
+        rows = range(r0, min(r0 + 256, n))
+        want, bound = _attention_rows(q, k[:, :kv], v[:, :kv], p0, rows)
+        bad = ~(np.abs(got[rows] - want) <= bound)
+        assert not bad.any(), (np.argwhere(bad)[:5] + [r0, 0, 0], np.abs(got[rows] - want)[bad].max())
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd,prompt,rows", [(16, 4, 64, 1555, 2048), (16, 2, 64, 3107, 1536),
                                                          (16, 16, 128, 1601, 2048)])
 @pytest.mark.parametrize("sharp", [1.0, 25.0])
 def test_prefill_attention_of_long_chunks(ctx, n_heads, n_kv, hd, prompt, rows, sharp):
     """Chunks of enough positions for the 128-query blocks of the prefill
-    attention (a partial last block, a second chunk behind 1536 cached
-    positions): the last position's logits against the oracle.  Its value
-    depends on every row of the first layer's attention.  `sharp` scales the
-    query projection, so that scores spread over many powers of two and the
+    attention, in a whole prompt: the last position's logits against the
+    oracle (test_attention_rows checks the kernel's every row).  `sharp` scales
+    the query projection, so that scores spread over many powers of two and the
     running maximum rises in steps larger than the kernel's rescaling
     threshold."""
     cfg = LlamaConfig(n_layers=2, hidden=n_heads * hd, n_heads=n_heads, n_kv_heads=n_kv, head_dim=hd,
