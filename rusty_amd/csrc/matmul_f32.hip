@@ -473,6 +473,12 @@ bool mfma_fits(int v, int64_t m, int64_t k, int64_t n, int num_cus) {
 //    24.8, 16x512x4096 5.0 -> 5.4; even at 16x4096x4096 25.4 -> 25.1);
 //  * over 256 k for a single 16x16 tile: the register-staged chains
 //    (1x4096x16 22.3 / 18.6 / 22.3 -> 24.4 / 24.2 / 42.2);
+//  * 9 to 16 columns over whole k-chunks where an operand loads by element (its
+//    rows no multiple of 4), up to 128 rows, or 2048 of k <= 1024: the
+//    register-staged chains (17x1024x9 8.0 / 8.1 -> 8.8 / 9.5 AB / ATB,
+//    17x4096x9 27.0 / 27.3 -> 27.8 / 30.9, A^T.B 101x1024x16 8.4 -> 9.2; with a
+//    ragged k, or more rows over a long k, the other way: 100x1022x9 10.3 -> 9.7 / 9.2,
+//    A^T.B 1001x4096x16 31.8 -> 29.6);
 //  * everything else: the matrix cores (4096^3 2270 / 2185 / 2223 -> 978 /
 //    998 / 966, 512x4096x4096 368 / 329 / 360 -> 146 / 146 / 139, 1024^3 74 /
 //    66 / 74 -> 21, 300x1000x777 72 / 64 / 72 -> 10.2 / 9.0 / 10.1,
@@ -485,9 +491,10 @@ Route route(int v, const TA *a, const float *b, int64_t m, int64_t k, int64_t n,
     const bool chain = k > 64 && chain_fits(m, k, n);
     if constexpr (std::is_same_v<TA, float>)
         if (chain && v == MM_ABT && m * n <= 65536 && ring_ok(a, b, k)) return ROUTE_RING;
-    const int64_t tiles = cdiv(m, 16) * cdiv(n, 16);
-    if (chain && k > 256 && tiles <= 1)
-        return ROUTE_CHAIN;
+    const bool one_tile = k > 256 && m <= 16 && n <= 16;
+    const bool by_element = n > 8 && n <= 16 && k % chain_kc<16>() == 0 && (m <= 128 || (k <= 1024 && m <= 2048)) &&
+                            !(vec_a(v, a, m, k) && vec_b(v, b, k, n));
+    if (chain && (one_tile || by_element)) return ROUTE_CHAIN;
     return mfma_fits(v, m, k, n, num_cus) ? ROUTE_MFMA : ROUTE_TILED;
 }
 

@@ -23,7 +23,9 @@ SHAPES = [(2, 2, 2), (1, 1024, 1024), (8, 1024, 1024), (65, 33, 70), (128, 256, 
           (1, 4097, 16), (5, 1000, 40), (33, 600, 9), (7, 300, 3), (2, 513, 100), (512, 4096, 16),
           (512, 200, 520), (1030, 64, 600),
           # 16-byte rows with ragged row and column blocks and a partial last chunk
-          (20, 520, 44), (12, 700, 36)]
+          (20, 520, 44), (12, 700, 36),
+          # 9 to 16 columns over whole k-chunks, rows no multiple of 4
+          (17, 1024, 9), (101, 1536, 16)]
 
 
 def _run(engine, ctx, op, a, b, m, n):

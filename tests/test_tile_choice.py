@@ -112,3 +112,16 @@ def test_gemm_tile_outside_the_fitted_times():
     assert gemm_tile(0, 1066, 2720, 1152) == (128, 128)
     assert gemm_tile(0, 157, 8448, 896) == (64, 64)  # 128x64 17.3 us, 64x64 8.5
     assert gemm_tile(1, 390, 4992, 1408) == (64, 64)
+
+
+def test_thin_products_that_load_by_element():
+    """9 to 16 columns over whole k-chunks with rows that are no multiple of 4
+    stay on the register-staged chains; ragged k and whole pieces do not."""
+    for variant, m, n in ((0, 17, 9), (0, 100, 9), (2, 17, 9), (2, 17, 16), (2, 101, 16)):
+        for k in (512, 1024, 4096):
+            assert matmul_kernel(variant, m, k, n) == 1
+        assert matmul_kernel(variant, m, 1022, n) == (32, 32) or variant == 2 and matmul_kernel(variant, m, 1022, n) != 1
+    assert matmul_kernel(2, 2001, 1024, 16) == 1 and matmul_kernel(2, 2001, 4096, 16) != 1
+    for variant, m, n in ((0, 100, 16), (2, 100, 16), (2, 500, 16), (0, 101, 16)):  # whole pieces
+        assert matmul_kernel(variant, m, 4096, n) not in (0, 1, 2)
+    assert matmul_kernel(2, 17, 4096, 8) != 1 and matmul_kernel(2, 17, 4096, 17) != 1
