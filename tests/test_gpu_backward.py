@@ -13,6 +13,7 @@ import pytest
 from conftest import f16_tol_check
 from oracle import oracle as orc
 from rusty_amd import DType, QuantizedTensor, RqError, UnifiedTensor, synth
+from tile_query import dx_kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -45,16 +46,35 @@ def test_dx_bit_exact_f32(ctx, engine, m, n_out, k_in, fmt):
                                               (5, 1028, 1100, 0), (1100, 68, 12, 12), (33, 60, 256, 128),
                                               (64, 64, 64, 64), (17, 30, 34, 0), (20, 40, 60, 24)])
 def test_dx_tiles_bit_exact(ctx, engine, m, n_out, k_in, grp):
-    """Every tile of the matrix-core kernel at ragged edges and partial last
-    stages, groups of one piece up, and the shapes it leaves to the VALU
-    kernel (widths not a multiple of 4, groups that do not divide k_in)."""
+    """The matrix-core kernel's 32x32 and 64x64 tiles at ragged edges and
+    partial last stages, groups of one piece up, and the shapes it leaves to
+    the VALU kernel (widths not a multiple of 4, groups that do not divide
+    k_in)."""
+    _check_dx(ctx, engine, m, n_out, k_in, grp, bias=grp != 32)
+
+
+# Every tile over more than seven stages and a partial last one: the weight's codes, scales and
+# biases move on stage by stage, ragged in rows and columns.
+@pytest.mark.parametrize("tile,m,n_out,k_in,grp,bias", [
+    ((16, 64), 8, 460, 11008, 0, False), ((16, 64), 7, 460, 11004, 4, True), ((64, 16), 11007, 460, 8, 0, False),
+    ((64, 16), 11007, 460, 8, 4, True), ((32, 32), 97, 460, 700, 0, False), ((32, 32), 97, 460, 704, 64, True),
+    ((64, 64), 40, 460, 11004, 0, False), ((64, 64), 511, 228, 4096, 64, True), ((64, 64), 511, 228, 4096, 128, False),
+    ((128, 128), 2501, 460, 1300, 0, False), ((128, 128), 2501, 460, 1300, 20, True),
+    (0, 1041, 28, 4104, 0, False), (0, 1041, 28, 4104, 8, True)])
+def test_dx_long_reductions_bit_exact(ctx, engine, tile, m, n_out, k_in, grp, bias):
+    """(tile 0: the short reductions that stay on the VALU kernel)"""
+    assert dx_kernel(1 if grp else 0, grp, m, n_out, k_in) == tile
+    _check_dx(ctx, engine, m, n_out, k_in, grp, bias)
+
+
+def _check_dx(ctx, engine, m, n_out, k_in, grp, bias):
     g = synth.rng(m + n_out + k_in)
     if not grp:
         q, s = synth.rowwise_weight(g, n_out, k_in)
         w, wdeq = QuantizedTensor.rowwise(ctx, q, s), orc.rowwise_dequantize(q, s)
     else:
         u, s, b = synth.affine_weight(g, n_out, k_in, group=grp)
-        b = None if grp == 32 else b
+        b = b if bias else None
         w = QuantizedTensor.affine(ctx, u, s, b, group=grp)
         wdeq = orc.affine_dequantize(u, s, np.zeros_like(s) if b is None else b, group=grp)
     for dt in (np.float32, np.float16):

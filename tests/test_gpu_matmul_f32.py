@@ -12,6 +12,7 @@ import pytest
 
 from oracle import oracle as orc
 from rusty_amd import UnifiedTensor
+from tile_query import matmul_kernel
 
 pytestmark = pytest.mark.gpu
 
@@ -69,9 +70,9 @@ def test_shape_mismatch_raises(ctx, engine):
         engine.matmul(ctx, A, B, out)
 
 
-# The matrix-core kernel's tiles (128x128, 64x64, 32x32, 16x64, 64x16): outputs
-# one short of, at and past whole tiles, k below a stage (32 or 64), at whole
-# stages and one past, row pitches in whole 16-byte pieces and not.
+# The matrix-core kernel on its 32x32 and 64x64 tiles: outputs one short of, at
+# and past whole tiles, k below a stage (32 or 64), at whole stages and one past,
+# row pitches in whole 16-byte pieces and not (every tile over many stages: below).
 MFMA_SHAPES = [(2050, 52, 2052), (1920, 64, 2047), (1023, 33, 1025), (1000, 96, 1000), (255, 100, 255),
                (97, 65, 130), (64, 128, 64), (63, 127, 65), (15, 70, 1500), (16, 64, 4100), (1500, 70, 15),
                (2100, 129, 16), (33, 17, 31), (17, 18, 19), (1, 20, 300), (300, 21, 1)]
@@ -79,6 +80,20 @@ MFMA_SHAPES = [(2050, 52, 2052), (1920, 64, 2047), (1023, 33, 1025), (1000, 96, 
 
 @pytest.mark.parametrize("m,k,n", MFMA_SHAPES)
 def test_matrix_core_tiles_bit_exact(ctx, engine, m, k, n):
+    test_matmul_family_bit_exact(ctx, engine, m, k, n)
+
+
+# Every tile over more than seven stages (the ring of three turns twice, registers refill) and a
+# partial last one, ragged in rows and columns; operands in whole 16-byte pieces and by element.
+LONG_SHAPES = [((16, 64), 8, 460, 11008), ((16, 64), 9, 461, 11009), ((64, 16), 11008, 460, 8),
+               ((64, 16), 11009, 461, 9), ((32, 32), 100, 460, 1100), ((32, 32), 101, 461, 1099),
+               ((64, 64), 40, 460, 11008), ((64, 64), 41, 461, 11009), ((128, 128), 2500, 460, 1300),
+               ((128, 128), 2501, 461, 1301)]
+
+
+@pytest.mark.parametrize("tile,m,k,n", LONG_SHAPES)
+def test_matrix_core_long_reductions_bit_exact(ctx, engine, tile, m, k, n):
+    assert [matmul_kernel(v, m, k, n) for v in range(3)] == [tile] * 3
     test_matmul_family_bit_exact(ctx, engine, m, k, n)
 
 

@@ -17,6 +17,7 @@ import pytest
 from conftest import f16_tol_check, f32_norm_check
 from oracle import oracle as orc
 from rusty_amd import DType, QuantizedTensor, RqError, UnifiedTensor, synth
+from tile_query import gemm_tile
 
 pytestmark = pytest.mark.gpu
 
@@ -309,10 +310,9 @@ def test_config4_prefill(ctx, engine, n, k):
     _check_prefill(y, x, q, s, f"C4 2048x{n}x{k}")
 
 
-# tile per shape on a 256-CU device: 64x64 for the first, second and fourth, 128x64 for
-# (300, 4096), 128x128 (two k-groups of 4 waves, weight staged in pairs of k-steps) for
-# (770, 4096) and (1100, 4100), 128x256 (the same) for (1500, 4100); k = 1088 is 17 k-steps, not a
-# multiple of the LDS ring period, and odd (the last weight pair is half past the k range)
+# ragged rows and columns: 64x64 tiles for the first four, 64x128 for (770, 4096), 192x128 for
+# (1100, 4100), 128x256 for the 1500-row ones; k = 1088 is 17 k-steps, not a multiple of the LDS
+# ring period, and odd (the last weight pair is half past the k range).  Every tile by name: below
 @pytest.mark.parametrize("m,n,k", [(17, 300, 1024), (200, 136, 2048), (300, 4096, 64), (129, 129, 128),
                                    (770, 4096, 128), (1500, 4100, 64), (1100, 4100, 1088), (1500, 4100, 1088)])
 def test_gemm_ragged(ctx, engine, m, n, k):
@@ -324,13 +324,28 @@ def test_gemm_ragged(ctx, engine, m, n, k):
     assert ok, (max_abs, rel)
 
 
-# Every tile of the choice by fitted time (192x128 and 64x128 beside the power-of-two ones), with
-# a partial last row and column tile, k-steps odd and not a multiple of the ring period, both
-# formats and output types; rows at tile edges against the f64 truth.
+# The choice by fitted time, with a partial last row and column tile, k-steps odd and not a multiple
+# of the ring period, both formats and output types; rows at tile edges against the f64 truth.
 @pytest.mark.parametrize("m,n,k", [(1500, 4090, 128), (1345, 2300, 128), (1010, 4100, 1088), (600, 2600, 192),
                                    (130, 4000, 2048), (250, 4100, 1088), (385, 3000, 320)])
 @pytest.mark.parametrize("fmt", [0, 1])
 def test_gemm_tile_choice(ctx, engine, m, n, k, fmt):
+    _check_gemm_rows(ctx, engine, m, n, k, fmt)
+
+
+# Every tile of either format over at least 17 k-steps, so that the 4- and 6-stage X rings and
+# the weight-pair ring refill several times (an odd last step among them).
+@pytest.mark.parametrize("fmt,tile,m,n,k", [
+    (0, (64, 64), 67, 7000, 1088), (0, (128, 64), 507, 4090, 4160), (0, (64, 128), 385, 8990, 1088),
+    (0, (128, 128), 200, 8990, 1088), (0, (192, 128), 385, 9990, 1088), (0, (128, 256), 600, 8990, 1088),
+    (1, (64, 64), 67, 7000, 1088), (1, (128, 64), 507, 4090, 2112), (1, (64, 128), 385, 8990, 1088),
+    (1, (128, 128), 200, 8990, 1088), (1, (192, 128), 530, 6990, 1088), (1, (128, 256), 600, 8990, 1088)])
+def test_gemm_every_tile_long_k(ctx, engine, fmt, tile, m, n, k):
+    assert gemm_tile(fmt, m, n, k) == tile
+    _check_gemm_rows(ctx, engine, m, n, k, fmt)
+
+
+def _check_gemm_rows(ctx, engine, m, n, k, fmt):
     g = synth.rng(m + n + k + fmt)
     if fmt:
         u, s, b = synth.affine_weight(g, n, k)
@@ -483,7 +498,7 @@ def test_config4_prefill_f32_activations(ctx, engine):
 # epilogue multiplies back, so rows with entries of 1e5..3e5 (fp16 ends at
 # 65504) and a row of values ~1e-6 (below fp16's normal range) are held to the
 # fp16 bar of their own rows against the f64 truth of the f32 input;
-# 300 tokens: 128x64 tiles, 40 tokens: split-K 64x64 tiles.
+# 64x64 tiles, unsplit at 300 tokens, split-K at 40.
 @pytest.mark.parametrize("m,n,k,fmt", [(300, 1024, 4096, 0), (40, 4096, 4096, 0), (300, 1024, 4096, 1)])
 def test_gemm_f32_activations_past_fp16_range(ctx, engine, m, n, k, fmt):
     g = synth.rng(9100 + m + fmt)
@@ -509,13 +524,13 @@ def test_gemm_f32_activations_past_fp16_range(ctx, engine, m, n, k, fmt):
     report(f"f32 x past fp16 range {m}x{n}x{k} fmt={fmt}: worst row max|dy|/max|y|", worst, worst)
 
 
-# every tile, split-K, group 128, and f32 activations in two chunks of the preparation area
+# split-K, group 128, and f32 activations in two chunks of the preparation area
 # (3000 x 16384 f32 -> fp16 is 98 MB: two chunks)
 @pytest.mark.parametrize("m,n,k,fmt,group,xdt", [
     (17, 300, 1024, 1, 64, np.float16),     # 64x64, split-K
     (9, 4096, 4096, 1, 64, np.float32),     # 9 tokens, f32: the GEMM (split-K)
     (100, 1000, 1088, 1, 64, np.float32),   # 64x64, 17 k-steps
-    (300, 4096, 1024, 1, 128, np.float16),  # 128x64, group 128
+    (300, 4096, 1024, 1, 128, np.float16),  # 64x64, group 128
     (770, 4096, 128, 1, 64, np.float32),    # 128x128 pairs
     (1500, 4100, 1088, 1, 64, np.float16),  # 128x256 pairs, odd k-step count
     (1500, 4100, 1024, 0, 0, np.float32),   # rowwise, f32 activations

@@ -13,6 +13,7 @@ import pytest
 from conftest import f16_tol_check
 from oracle import oracle as orc
 from rusty_amd import DType, QuantizedTensor, UnifiedTensor, synth
+from tile_query import gemm_tile
 
 pytestmark = pytest.mark.gpu
 
@@ -134,7 +135,7 @@ def test_swiglu_prefill_fused(ctx, engine, m, inter, hidden):
     assert ok
 
 
-@pytest.mark.parametrize("m,inter,hidden", [(1000, 2760, 1024), (768, 2816, 1024)], ids=["128x256", "128x128"])
+@pytest.mark.parametrize("m,inter,hidden", [(1000, 2760, 1024), (768, 2816, 1024)], ids=["128x256", "192x128"])
 def test_swiglu_prefill_fused_affine(ctx, engine, m, inter, hidden):
     """The fused gate/up GEMM on the reference's affine u8 weights (scale tables
     prepared at load): the tile's gate half stages its scales and offsets from
@@ -173,13 +174,30 @@ def test_swiglu_prefill_fused_tiles(ctx, engine, m, inter, hidden):
     """The fused gate/up product on the 64x128 and 192x128 tiles with partial
     last tiles (in rows, and in the columns of both halves): h at tile-edge
     rows against the f64 truth, both weight formats."""
+    _check_fused_h(ctx, engine, m, inter, hidden, (0, 1))
+
+
+# Every tile of the fused product over 17 k-steps: the 4-stage X ring and the weight-pair ring
+# refill several times, and the last weight pair is half past the k range.
+@pytest.mark.parametrize("fmt,tile,m,inter", [
+    (0, (64, 128), 300, 5632), (0, (128, 128), 67, 9000), (0, (192, 128), 385, 5000), (0, (128, 256), 200, 9000),
+    (1, (64, 128), 300, 5632), (1, (128, 128), 67, 9000), (1, (192, 128), 130, 10008), (1, (128, 256), 200, 9000)])
+def test_swiglu_prefill_every_tile_long_k(ctx, engine, fmt, tile, m, inter):
+    assert gemm_tile(fmt, m, inter, 1088, pair=True) == tile
+    _check_fused_h(ctx, engine, m, inter, 1088, (fmt,))
+
+
+def _check_fused_h(ctx, engine, m, inter, hidden, fmts):
     g = synth.rng(77 + m)
     x = synth.activations(g, m, hidden, sigma=0.5)
     rows = np.unique(np.r_[0, 1, np.minimum(np.arange(63, m, 64), m - 1), m - 1])
     wg, sg, wu, su, wd, sd = weights(g, inter, hidden)
-    _, h = run_mlp(ctx, engine, x, wg, sg, wu, su, wd, sd, ydt=np.float32)
-    _, _, ok = f16_tol_check(h[rows], h_truth(x[rows], wg, sg, wu, su))
-    assert ok and np.isfinite(h).all()
+    if 0 in fmts:
+        _, h = run_mlp(ctx, engine, x, wg, sg, wu, su, wd, sd, ydt=np.float32)
+        _, _, ok = f16_tol_check(h[rows], h_truth(x[rows], wg, sg, wu, su))
+        assert ok and np.isfinite(h).all()
+    if 1 not in fmts:
+        return
     ug, sg, bg = synth.affine_weight(g, inter, hidden)
     uu, su, bu = synth.affine_weight(g, inter, hidden)
     G, U = QuantizedTensor.affine(ctx, ug, sg, bg), QuantizedTensor.affine(ctx, uu, su, bu)
