@@ -350,16 +350,19 @@ __global__ __launch_bounds__(NW * 64) void k_attn_prefill(const _Float16 *__rest
 // fragments come from the row-major V tile by transposing reads
 // (ds_read_b64_tr_b16: 16 lanes take a block of 4 keys x 16 dims and each gets
 // one dim's 4 keys), in the key order the score accumulators hold P in.
+// P goes to the matrix cores as two fp16 terms, P = hi + lo to 2^-22: with one
+// term, over one running maximum per query (k_attn_prefill has one per wave, each
+// making a large weight exactly 1), rows lay up to 29 % further from float64
+// than k_attn_prefill's (relative 2-norm, scores of unit to 25-fold spread); with two
+// they are 0.3 to 32 % nearer, at what rounding the output alone costs.
 // The softmax is what bounds it: per score one max, one fma into the exponent,
-// one quarter-rate exp2, one add and half a conversion, against 16 matrix
-// instructions per 64 keys (counters at 2048 queries after 2048 cached
-// positions: VALU issuing 76 % of the cycles, matrix cores 28 %).  So the rest
-// is kept off every tile: scale and maximum enter the exponent's fma, the mask
-// runs on a wave's last tile only, and the accumulators are rescaled only when
-// some query's maximum passed the one they are relative to by 2^8 (P then
-// reaches 256, in fp16 to the same relative precision; sums are f32).
-// 4096 positions in two chunks, 32 heads of 64, per layer: 304 -> 120 us (573
-// TFLOP/s of the causal work).
+// one quarter-rate exp2, one add, a conversion and the residual's two, against
+// 24 matrix instructions per 64 keys.  So the rest is kept off every tile:
+// scale and maximum enter the exponent's fma, the mask runs on a wave's last
+// tile only, and the accumulators are rescaled only when some query's maximum
+// passed the one they are relative to by 2^8 (P then reaches 256; sums are f32).
+// 4096 positions in two chunks of 2048, 32 heads of 64, us per layer: 267
+// k_attn_prefill, 136 here (105 with one term for P).
 template <int HD>
 __global__ __launch_bounds__(256, 2) void k_attn_prefill_rows(const _Float16 *__restrict__ q, const _Float16 *__restrict__ kc,
                                                            const _Float16 *__restrict__ vc, _Float16 *__restrict__ out,
@@ -416,7 +419,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_rows(const _Float16 *__
     dma(0);
     dma(1);
     const int qpos = p0 + q0 + col;
-    // scores in log2 units (see above): p = 2^(c s - c m)
+    // scores in log2 units (see above): P = 2^(c s - c m)
     const float c = 1.4426950408889634f / sqrtf((float)HD);
     float m_run = -__builtin_inff(), l_run = 0.0f;
     floatx16 o[DT];
@@ -436,6 +439,8 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_rows(const _Float16 *__
             const int r = kr + 8 * e, ch = 4 * d + 2 * ((lane >> 4) & 1) + (i16 & 3) / 2;
             va[d][e] = (uint32_t)(r * ROW + ((ch ^ fv(r)) * 16) + (i16 & 1) * 8);
         }
+    typedef float float2v __attribute__((ext_vector_type(2)));
+    typedef _Float16 half2v __attribute__((ext_vector_type(2)));
     typedef short short4v __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) short4v lds_short4;
     typedef __attribute__((address_space(3))) half8 lds_half8;
@@ -484,15 +489,22 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_rows(const _Float16 *__
                 for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
         }
         const float mc = m_run * c;
-        half8 pf[4];
+        half8 pf[4], pl[4];  // P = pf + pl
         float ls[2] = {0.0f, 0.0f};
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc.t[t][r], c, -mc));
-                ls[r & 1] += pr;
-                pf[2 * t + (r >> 3)][r & 7] = (_Float16)pr;
+            for (int r = 0; r < 16; r += 2) {
+                const float2v pr = {__builtin_amdgcn_exp2f(__builtin_fmaf(sc.t[t][r], c, -mc)),
+                                    __builtin_amdgcn_exp2f(__builtin_fmaf(sc.t[t][r + 1], c, -mc))};
+                ls[0] += pr.x;
+                ls[1] += pr.y;
+                const half2v hi = __builtin_convertvector(pr, half2v);
+                const half2v lo = __builtin_convertvector((float2v{__builtin_fmaf((float)hi.x, -1.0f, pr.x), __builtin_fmaf((float)hi.y, -1.0f, pr.y)}), half2v);
+                pf[2 * t + (r >> 3)][r & 7] = hi.x;
+                pf[2 * t + (r >> 3)][(r & 7) + 1] = hi.y;
+                pl[2 * t + (r >> 3)][r & 7] = lo.x;
+                pl[2 * t + (r >> 3)][(r & 7) + 1] = lo.y;
             }
         l_run += ls[0] + ls[1];
 #pragma unroll
@@ -504,6 +516,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_rows(const _Float16 *__
                 const short4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16(pb + s2 * 16 * ROW / 8);
                 const uint2 ua = __builtin_bit_cast(uint2, a), ub = __builtin_bit_cast(uint2, b);
                 const half8 vf = __builtin_bit_cast(half8, make_uint4(ua.x, ua.y, ub.x, ub.y));
+                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl[s2], o[d], 0, 0, 0);
                 o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[s2], o[d], 0, 0, 0);
             }
         }
@@ -576,10 +589,9 @@ int launch_attn_prefill(const _Float16 *q, const _Float16 *kc, const _Float16 *v
     if (p0 % 32 != 0 || n < 1 || (hd != 64 && hd != 128) || n_heads % n_kv != 0) return RQ_ERR_UNSUPPORTED;
     // Blocks of 128 queries where they cover three quarters of the CUs (256 CUs, us
     // per layer, small blocks -> these, after 0 / 2048 / 6144 cached positions: 32 heads of 64,
-    // 768 positions (192 blocks) 20.1 -> 13.0, 61 -> 38, 148 -> 101, 2048 77 -> 32,
-    // 190 -> 72, 415 -> 153; 64 heads of 128, 257 positions (192 blocks, a third
-    // of them with one query) 23.7 -> 11.7, 130 -> 57, 341 -> 148; 32 heads of 64, 512
-    // positions (128 blocks), in a 4-layer prompt: 389 against 397).
+    // 768 positions (192 blocks) 21.2 -> 16.5, 61 -> 49, 148 -> 127, 2048 77 -> 41,
+    // 190 -> 96, 416 -> 206; 64 heads of 128, 257 positions (192 blocks, a third
+    // of them with one query) 23.2 -> 13.3, 129 -> 69, 341 -> 181).
     const int blocks = n_heads * ((n + 127) / 128);
     if (4 * blocks >= 3 * num_cus) {
         if (hd == 64)
