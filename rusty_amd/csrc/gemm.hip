@@ -1239,7 +1239,7 @@ int launch_gemm_qkv_rope(const rq_qweight &w, const _Float16 *x, int64_t m, cons
     const double pass = 2.0 + 6e-6 / 4.5 * (double)m * (double)N;
     if (std::min(a, b) > tile_cost(choose_tile(fmt, m, N, K / 64, cus), fmt, m, N, K / 64, cus) + pass)
         return RQ_ERR_UNSUPPORTED;
-    if (a < b)
+    if (a < 0.95 * b)  // nearly even: 64x64 (512 positions at 2560x2048 affine 424 us for 4 layers, 433)
         return launch_tiled<128, 64, true, 6, 4, 2, 2>(w, sc, fmt, x, q, RQ_F16, m, 4, cus, ws, s, GemmPair{}, &ro);
     return launch_tiled<64, 64, true, 4, 4, 2, 2>(w, sc, fmt, x, q, RQ_F16, m, 4, cus, ws, s, GemmPair{}, &ro);
 }
