@@ -387,10 +387,10 @@ def ops_bench(ctx, engine, use_graph: bool = True) -> list:
     after >= 0.25 s of warm-up replays, median of 3) against its roofline:
       dequantize          a2, kernels.wgsl:153-166: 1 B read + 4 B written per element
       affine_dequantize   a1, kernels.wgsl:379-400: + 8 B (scale, bias) per 64 elements
-      matmul_f32          a3, kernels.wgsl:7-54: 2 m k n flops, fp32 VALU; at configs[0]'s few
+      matmul_f32          a3, kernels.wgsl:7-54: 2 m k n flops, f32 matrix cores; at configs[0]'s few
                           outputs the bound is the k-long dependent fma chain of each output,
                           reported as the one-launch time of one wave's chain of k fmas
-      qmatmul_dx          f-4, MatMulNode::backward: dX = dY . deq(W), 2 m n k flops, fp32 VALU
+      qmatmul_dx          f-4, MatMulNode::backward: dX = dY . deq(W), 2 m n k flops, f32 matrix cores
       qmatmul_lora        a7 with an adapter, lib.rs:69-83: the fused product plus (x.A).B
     The dequantize kernels rotate 8 inputs and 4 outputs (384 MB, past the
     256 MB Infinity Cache)."""
