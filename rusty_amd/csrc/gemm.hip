@@ -1069,7 +1069,9 @@ double tile_cost(int id, int fmt, int64_t m, int64_t N, int64_t nk, int64_t cus)
                       c.next * (double)(full + (rem > 0) - 1);
     const double fill = (double)tiles / (double)(per * cus);
     // 64x128 reads the most bytes per product beside 64x64: 8 % for operands
-    // and outputs that do not stay in the caches the fit had them in
+    // and outputs that do not stay in the caches the fit had them in.  (Over 60
+    // random shapes on every tile 0.25 to 0.35 above chooses best; 2 % instead of
+    // the 8, over 459 calls, is even on average, 0.88-1.15x on single ones.)
     return us * (1.0 - 0.35 * (1.0 - fill)) * (id == T64x128 ? 1.08 : 1.0);
 }
 
