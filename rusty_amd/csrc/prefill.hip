@@ -10,8 +10,8 @@
 //                       into the KV cache at positions p0..p0+S-1
 //   k_attn_prefill      causal GQA attention of the S queries over cache
 //                       positions 0..p0+S-1 on the matrix cores (short chunks)
-//   k_attn_prefill_rows the same for chunks that fill the device with blocks
-//                       of 128 queries
+//   k_attn_prefill_rows the same, bit for bit, for chunks that fill the device
+//                       with blocks of 64 or 128 queries
 //
 // Attention of short chunks (flash-style, four waves per (query tile of 32, head)):
 // the scores of a key tile are computed transposed, S^T = K . Q^T, with
@@ -29,6 +29,8 @@
 // pieces of a row of V^T in that key order.  Scores, softmax and the
 // accumulators are f32 (exponentials as 2^x on scores scaled by log2 e);
 // q, k, v and p enter the matrix cores as fp16.
+#include <type_traits>
+
 #include "common.hpp"
 #include "lds_dma.hpp"
 
@@ -342,44 +344,53 @@ __global__ __launch_bounds__(NW * 64) void k_attn_prefill(const _Float16 *__rest
     }
 }
 
-// The same attention for chunks long enough to fill the device with blocks
-// of 128 queries: four waves of 32 consecutive queries of one head walk the
-// same key tiles of 64, which pass through LDS once per block (DMA, a ring of
-// three stages, one barrier per tile) instead of once per 32 queries through
-// every wave's registers.  K fragments are 16-byte reads of swizzled rows; V^T
-// fragments come from the row-major V tile by transposing reads
-// (ds_read_b64_tr_b16: 16 lanes take a block of 4 keys x 16 dims and each gets
-// one dim's 4 keys), in the key order the score accumulators hold P in.
-// P goes to the matrix cores as two fp16 terms, P = hi + lo to 2^-22: with one
-// term, over one running maximum per query (k_attn_prefill has one per wave, each
-// making a large weight exactly 1), rows lay up to 29 % further from float64
-// than k_attn_prefill's (relative 2-norm, scores of unit to 25-fold spread); with two
-// they are 0.3 to 32 % nearer, at what rounding the output alone costs.
-// The softmax is what bounds it: per score one max, one fma into the exponent,
-// one quarter-rate exp2, one add, a conversion and the residual's two, against
-// 24 matrix instructions per 64 keys.  So the rest is kept off every tile:
-// scale and maximum enter the exponent's fma, the mask runs on a wave's last
-// tile only, and the accumulators are rescaled only when some query's maximum
-// passed the one they are relative to by 2^8 (P then reaches 256; sums are f32).
-// 4096 positions in two chunks of 2048, 32 heads of 64, us per layer: 267
-// k_attn_prefill, 136 here (105 with one term for P).
-template <int HD>
-__global__ __launch_bounds__(256, 2) void k_attn_prefill_rows(const _Float16 *__restrict__ q, const _Float16 *__restrict__ kc,
-                                                           const _Float16 *__restrict__ vc, _Float16 *__restrict__ out,
-                                                           int p0, int n, int n_heads, int n_kv, int max_seq) {
+// The same attention, bit for bit, for chunks long enough to fill the device
+// with blocks of several query tiles: their waves walk the same key tiles of
+// 64, which pass through LDS once per block (DMA, a ring of two or three stages,
+// one barrier per tile) instead of once per 32 queries through every wave's
+// registers.  K fragments are 16-byte reads of swizzled rows; V^T fragments come
+// from the row-major V tile by transposing reads (ds_read_b64_tr_b16: 16 lanes
+// take a block of 4 keys x 16 dims and each gets one dim's 4 keys), in the key
+// order the score accumulators hold P in.
+// Each query has the four partial softmaxes (running max, sum, unnormalised O)
+// that k_attn_prefill's four waves keep of their 32-key tiles w, w + 4, ...,
+// each updated with that kernel's operations in its order and combined in its
+// order: a row does not depend on the chunk length that chose the kernel.  (One
+// partial over all keys with a maximum that may lag, rescaled rarely, lay 1 to 29 %
+// further from float64: every running maximum gives one large weight as
+// exactly 1, and there are four; it took 72 us at 2048 queries after 2048
+// positions, this 83.)  TPW 32-key tiles of each 64 are a wave's:
+//  * TPW = 2: four query tiles per block, a wave keeps all four partials
+//    (head_dim 64: 128 accumulator registers, two waves per SIMD);
+//  * TPW = 1: two query tiles per block and two waves for each, with two
+//    partials (head_dim 64: three waves per SIMD; 128: two), joined through LDS.
+// The softmax is what bounds it: per score a multiplication, half a max, a
+// subtraction, one quarter-rate exp2, an addition and half a conversion, against
+// 16 matrix instructions per 64 keys at head_dim 64.  So the rest is kept off
+// every tile: the mask runs on a wave's last 32 keys only, and partials are
+// rescaled only when the maximum of one of their queries rose (the factor of the
+// others is exactly 1); a wave's two tiles are interleaved, as their chains of
+// matrix instructions, max, exchange and exponent are what it would wait for (one
+// after the other: 83 -> 92 us).
+template <int HD, int TPW>
+__global__ __launch_bounds__(256, HD == 64 && TPW == 1 ? 3 : 2) void k_attn_prefill_rows(
+    const _Float16 *__restrict__ q, const _Float16 *__restrict__ kc, const _Float16 *__restrict__ vc,
+    _Float16 *__restrict__ out, int p0, int n, int n_heads, int n_kv, int max_seq) {
+#pragma clang fp contract(off)
     constexpr int KS = HD / 16, DT = HD / 32;
     constexpr int ROW = HD * 2, CH = ROW / 16;  // bytes and 16-byte chunks per row
-    constexpr int KT = 64, NS = 3;
-    constexpr int TILE = KT * ROW;                   // one operand's tile
-    constexpr int UW = TILE / 1024 / 4;              // DMA units per wave and operand
-    constexpr int RPU = 1024 / ROW;                  // rows per unit
+    constexpr int KT = 64, NS = TPW == 2 ? 3 : 2;  // keys per tile, LDS stages
+    constexpr int QW = 2 * TPW, NP = 2 * TPW;      // query tiles per block, partials per wave
+    constexpr int TILE = KT * ROW;              // one operand's tile
+    constexpr int UW = TILE / 1024 / 4;         // DMA units per wave and operand
+    constexpr int RPU = 1024 / ROW;             // rows per unit
     __shared__ __attribute__((aligned(1024))) unsigned char lds[NS * 2 * TILE];
-    const int nqb = (n + 127) / 128;
+    const int nqb = (n + 32 * QW - 1) / (32 * QW);
     const int head = blockIdx.x % n_heads;
-    const int qb = (nqb - 1 - (int)blockIdx.x / n_heads) * 128;  // the longest first
+    const int qb = (nqb - 1 - (int)blockIdx.x / n_heads) * (32 * QW);  // the longest first
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 31, hf = lane >> 5;
-    const int q0 = qb + 32 * wv;
+    const int pg = TPW == 2 ? 0 : wv & 1, q0 = qb + 32 * (TPW == 2 ? wv : wv >> 1);
     const int g = head / (n_heads / n_kv);
     const int kv_len = p0 + n;
     const auto rk = make_rsrc_s(kc + (size_t)g * max_seq * HD, (uint32_t)kv_len * ROW);
@@ -397,9 +408,9 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_rows(const _Float16 *__
         koff[u] = (uint32_t)(r * ROW + ((c ^ fk(r)) * 16));
         voff[u] = (uint32_t)(r * ROW + ((c ^ fv(r)) * 16));
     }
-    const int last_b = min(p0 + qb + 127, kv_len - 1);
-    const int ntiles = last_b / KT + 1;                                 // of the block
-    const int mine = q0 < n ? min(p0 + q0 + 31, kv_len - 1) / KT + 1 : 0;  // of this wave
+    const int last_b = min(p0 + qb + 32 * QW - 1, kv_len - 1);
+    const int ntiles = last_b / KT + 1;                                    // of the block
+    const int mine = q0 < n ? min(p0 + q0 + 31, kv_len - 1) / 32 + 1 : 0;  // 32-key tiles of this wave
     const uint32_t lds0 = lds_addr(&lds[0]);
     auto dma = [&](int kt) {
         const bool live = kt < ntiles;
@@ -416,17 +427,21 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_rows(const _Float16 *__
         const uint32_t off = q0 + col < n ? (((uint32_t)(q0 + col) * n_heads + head) * HD + 16 * s + 8 * hf) * 2u : kOOB;
         qf[s] = __builtin_bit_cast(half8, bload(rq, off));
     }
-    dma(0);
-    dma(1);
+#pragma unroll
+    for (int kt = 0; kt < NS - 1; ++kt) dma(kt);
     const int qpos = p0 + q0 + col;
-    // scores in log2 units (see above): P = 2^(c s - c m)
-    const float c = 1.4426950408889634f / sqrtf((float)HD);
-    float m_run = -__builtin_inff(), l_run = 0.0f;
-    floatx16 o[DT];
+    const float scale = 1.4426950408889634f / sqrtf((float)HD);  // scores in log2 units
+    float m_run[NP], l_run[NP];
+    floatx16 o[NP][DT];
 #pragma unroll
-    for (int d = 0; d < DT; ++d)
+    for (int w = 0; w < NP; ++w) {
+        m_run[w] = -__builtin_inff();
+        l_run[w] = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+        for (int d = 0; d < DT; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[w][d][r] = 0.0f;
+    }
     // LDS byte offsets of this lane's reads within a tile
     uint32_t ka[KS], va[DT][2];
 #pragma unroll
@@ -439,115 +454,167 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_rows(const _Float16 *__
             const int r = kr + 8 * e, ch = 4 * d + 2 * ((lane >> 4) & 1) + (i16 & 3) / 2;
             va[d][e] = (uint32_t)(r * ROW + ((ch ^ fv(r)) * 16) + (i16 & 1) * 8);
         }
-    typedef float float2v __attribute__((ext_vector_type(2)));
-    typedef _Float16 half2v __attribute__((ext_vector_type(2)));
     typedef short short4v __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) short4v lds_short4;
     typedef __attribute__((address_space(3))) half8 lds_half8;
-    struct Scores {
-        floatx16 t[2];  // [t][r]: key 64 kt + 32 t + 8 (r / 4) + 4 hf + r % 4 against query qpos
+    // scores of 32-key tile j: sc[r]: key 32 j + 8 (r / 4) + 4 hf + r % 4 against query qpos
+    auto scores = [&](int j, floatx16 &sc) {
+        const uint32_t kb = lds0 + (uint32_t)((j >> 1) % NS) * (2 * TILE) + (uint32_t)(j & 1) * (32 * ROW);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[r] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const lds_half8 *)(kb + ka[s]), qf[s], sc, 0, 0, 0);
     };
-    auto scores = [&](int kt, Scores &sc) {
-        const uint32_t kb = lds0 + (uint32_t)(kt % NS) * (2 * TILE);
+    // scores, softmax and P . V of the N 32-key tiles from j on into partials W, W + 1,
+    // the two interleaved
+    auto keys = [&](auto n_c, auto w_c, int j) {
+#pragma clang fp contract(off)
+        constexpr int N = decltype(n_c)::value, W = decltype(w_c)::value;
+        floatx16 sc[N];
+        float m_new[N], alpha[N];
+        bool rose = false;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int i = 0; i < N; ++i) scores(j + i, sc[i]);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sc.t[t][r] = 0.0f;
+        for (int i = 0; i < N; ++i) {
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const lds_half8 *kp = (const lds_half8 *)(kb + ka[s]);
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-                sc.t[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kp[t * 32 * ROW / 16], qf[s], sc.t[t], 0, 0, 0);
-        }
-    };
-    auto weigh = [&](int kt, Scores &sc) {  // softmax and P . V of tile kt
-        const uint32_t vb = lds0 + (uint32_t)(kt % NS) * (2 * TILE) + TILE;
-        if (kt == mine - 1) {
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
+            for (int r = 0; r < 16; ++r) sc[i][r] = sc[i][r] * scale;
+            if (j + i == mine - 1) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int key = KT * kt + 32 * t + 8 * (r >> 2) + 4 * hf + (r & 3);
-                    sc.t[t][r] = key <= qpos ? sc.t[t][r] : -__builtin_inff();
+                    const int key = 32 * (j + i) + 8 * (r >> 2) + 4 * hf + (r & 3);
+                    sc[i][r] = key <= qpos ? sc[i][r] : -__builtin_inff();
                 }
-        }
-        float mt = sc.t[0][0];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sc.t[t][r]);
-        mt = fmaxf(mt, __shfl_xor(mt, 32));
-        if (__builtin_amdgcn_ballot_w64((mt - m_run) * c > 8.0f)) {
-            const float m_new = fmaxf(m_run, mt);
-            const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * c);
-            m_run = m_new;
-            l_run *= alpha;
-#pragma unroll
-            for (int d = 0; d < DT; ++d)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
-        }
-        const float mc = m_run * c;
-        half8 pf[4], pl[4];  // P = pf + pl
-        float ls[2] = {0.0f, 0.0f};
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                const float2v pr = {__builtin_amdgcn_exp2f(__builtin_fmaf(sc.t[t][r], c, -mc)),
-                                    __builtin_amdgcn_exp2f(__builtin_fmaf(sc.t[t][r + 1], c, -mc))};
-                ls[0] += pr.x;
-                ls[1] += pr.y;
-                const half2v hi = __builtin_convertvector(pr, half2v);
-                const half2v lo = __builtin_convertvector((float2v{__builtin_fmaf((float)hi.x, -1.0f, pr.x), __builtin_fmaf((float)hi.y, -1.0f, pr.y)}), half2v);
-                pf[2 * t + (r >> 3)][r & 7] = hi.x;
-                pf[2 * t + (r >> 3)][(r & 7) + 1] = hi.y;
-                pl[2 * t + (r >> 3)][r & 7] = lo.x;
-                pl[2 * t + (r >> 3)][(r & 7) + 1] = lo.y;
             }
-        l_run += ls[0] + ls[1];
+            float mt = sc[i][0];
+#pragma unroll
+            for (int r = 1; r < 16; ++r) mt = fmaxf(mt, sc[i][r]);
+            m_new[i] = fmaxf(m_run[W + i], fmaxf(mt, __shfl_xor(mt, 32)));
+            alpha[i] = 1.0f;
+            rose = rose || m_new[i] != m_run[W + i];
+        }
+        if (__builtin_amdgcn_ballot_w64(rose)) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                alpha[i] = __builtin_amdgcn_exp2f(m_run[W + i] - m_new[i]);
+                m_run[W + i] = m_new[i];
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) o[W + i][d][r] *= alpha[i];
+            }
+        }
+        half8 pf[N][2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const float pr = __builtin_amdgcn_exp2f(sc[i][r] - m_run[W + i]);
+                l_run[W + i] = r == 0 ? __builtin_fmaf(l_run[W + i], alpha[i], pr) : l_run[W + i] + pr;
+                pf[i][r >> 3][r & 7] = (_Float16)pr;
+            }
+        const uint32_t vb = lds0 + (uint32_t)((j >> 1) % NS) * (2 * TILE) + TILE + (uint32_t)(j & 1) * (32 * ROW);
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
             lds_short4 *pa = (lds_short4 *)(vb + va[d][0]), *pb = (lds_short4 *)(vb + va[d][1]);
 #pragma unroll
-            for (int s2 = 0; s2 < 4; ++s2) {
-                const short4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(pa + s2 * 16 * ROW / 8);
-                const short4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16(pb + s2 * 16 * ROW / 8);
-                const uint2 ua = __builtin_bit_cast(uint2, a), ub = __builtin_bit_cast(uint2, b);
-                const half8 vf = __builtin_bit_cast(half8, make_uint4(ua.x, ua.y, ub.x, ub.y));
-                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pl[s2], o[d], 0, 0, 0);
-                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[s2], o[d], 0, 0, 0);
-            }
+            for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    const short4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(pa + (2 * i + s2) * 16 * ROW / 8);
+                    const short4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16(pb + (2 * i + s2) * 16 * ROW / 8);
+                    const uint2 ua = __builtin_bit_cast(uint2, a), ub = __builtin_bit_cast(uint2, b);
+                    const half8 vf = __builtin_bit_cast(half8, make_uint4(ua.x, ua.y, ub.x, ub.y));
+                    o[W + i][d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[i][s2], o[W + i][d], 0, 0, 0);
+                }
         }
     };
-    // The scores of tile kt + 1 are multiplied while tile kt's softmax runs.
-    Scores sc[2];
-    wait_vmcnt<2 * UW>();
-    __syncthreads();
-    if (mine > 0) scores(0, sc[0]);
-    for (int kt = 0; kt < ntiles; kt += 2) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            // tile kt + u + 1 has landed, and every wave is done with tile kt + u - 1
-            wait_vmcnt<0>();
-            __syncthreads();
-            dma(kt + u + 2);
-            if (kt + u + 1 < mine) scores(kt + u + 1, sc[1 - u]);
-            if (kt + u < mine) weigh(kt + u, sc[u]);
+    auto step = [&](auto u_c, int kt) {
+        constexpr int U = decltype(u_c)::value;
+        // tile kt has landed, and every wave is done with the one whose stage the next takes
+        wait_vmcnt<(NS - 2) * 2 * UW>();
+        __syncthreads();
+        dma(kt + NS - 1);
+        const int j = 2 * kt + pg;
+        if constexpr (TPW == 2) {
+            if (j + 1 < mine) keys(std::integral_constant<int, 2>{}, std::integral_constant<int, 2 * U>{}, j);
+            else if (j < mine) keys(std::integral_constant<int, 1>{}, std::integral_constant<int, 2 * U>{}, j);
+        } else {
+            if (j < mine) keys(std::integral_constant<int, 1>{}, std::integral_constant<int, U>{}, j);
         }
+    };
+    for (int kt = 0; kt < ntiles; kt += 2) {
+        step(std::integral_constant<int, 0>{}, kt);
+        step(std::integral_constant<int, 1>{}, kt + 1);
     }
     wait_vmcnt<0>();  // no DMA in flight past this point
+    // The four partials of every query, combined in k_attn_prefill's order; with two
+    // waves per query tile (partials 0 and 2, 1 and 3) through LDS.
+    float ms[4], ls[4];
+    float *co = reinterpret_cast<float *>(lds) + (q0 - qb) / 32 * (TPW == 2 ? 0 : 2 * DT * 16 * 64);
+    if constexpr (TPW == 1) {
+        __shared__ float cml[QW][2][2][64];
+        float(&ml)[2][2][64] = cml[(q0 - qb) / 32];
+        __syncthreads();  // every wave is done with the ring
+        if (pg) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                ml[u][0][lane] = m_run[u];
+                ml[u][1][lane] = l_run[u];
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) co[((u * DT + d) * 16 + r) * 64 + lane] = o[u][d][r];
+            }
+        }
+        __syncthreads();
+        if (pg) return;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            ms[2 * u] = m_run[u];
+            ls[2 * u] = l_run[u];
+            ms[2 * u + 1] = ml[u][0][lane];
+            ls[2 * u + 1] = ml[u][1][lane];
+        }
+    } else {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            ms[w] = m_run[w];
+            ls[w] = l_run[w];
+        }
+    }
+    float mx = ms[0];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) mx = fmaxf(mx, ms[w]);
+    float wt[4], L = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        wt[w] = __builtin_amdgcn_exp2f(ms[w] - mx);
+        L = __builtin_fmaf(wt[w], ls[w] + __shfl_xor(ls[w], 32), L);  // both halves of the query's keys
+    }
+    const float inv = 1.0f / L;
     if (q0 + col >= n) return;
-    const float inv = 1.0f / (l_run + __shfl_xor(l_run, 32));
     _Float16 *orow = out + ((size_t)(q0 + col) * n_heads + head) * HD;
     typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 #pragma unroll
     for (int d = 0; d < DT; ++d)
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
-            const half4 v = {(_Float16)(o[d][4 * r4] * inv), (_Float16)(o[d][4 * r4 + 1] * inv),
-                             (_Float16)(o[d][4 * r4 + 2] * inv), (_Float16)(o[d][4 * r4 + 3] * inv)};
+            half4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = 4 * r4 + e;
+                float a = 0.0f;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    float ow;
+                    if constexpr (TPW == 2) ow = o[w][d][r];
+                    else ow = w & 1 ? co[((w / 2 * DT + d) * 16 + r) * 64 + lane] : o[w / 2][d][r];
+                    a = __builtin_fmaf(wt[w], ow, a);
+                }
+                v[e] = (_Float16)(a * inv);
+            }
             *reinterpret_cast<half4 *>(orow + 32 * d + 8 * r4 + 4 * hf) = v;
         }
 }
@@ -587,19 +654,25 @@ int launch_rope_scatter(const float *qkv, const float2 *rope, int p0, int n, int
 int launch_attn_prefill(const _Float16 *q, const _Float16 *kc, const _Float16 *vc, _Float16 *out, int p0, int n,
                         int n_heads, int n_kv, int hd, int max_seq, int num_cus, hipStream_t s) {
     if (p0 % 32 != 0 || n < 1 || (hd != 64 && hd != 128) || n_heads % n_kv != 0) return RQ_ERR_UNSUPPORTED;
-    // Blocks of 128 queries where they cover three quarters of the CUs (256 CUs, us
-    // per layer, small blocks -> these, after 0 / 2048 / 6144 cached positions: 32 heads of 64,
-    // 768 positions (192 blocks) 21.2 -> 16.5, 61 -> 49, 148 -> 127, 2048 77 -> 41,
-    // 190 -> 96, 416 -> 206; 64 heads of 128, 257 positions (192 blocks, a third
-    // of them with one query) 23.2 -> 13.3, 129 -> 69, 341 -> 181).
-    const int blocks = n_heads * ((n + 127) / 128);
-    if (4 * blocks >= 3 * num_cus) {
-        if (hd == 64)
-            hipLaunchKernelGGL((k_attn_prefill_rows<64>), dim3((unsigned)blocks), dim3(256), 0, s, q, kc, vc, out, p0,
-                               n, n_heads, n_kv, max_seq);
-        else
-            hipLaunchKernelGGL((k_attn_prefill_rows<128>), dim3((unsigned)blocks), dim3(256), 0, s, q, kc, vc, out, p0,
-                               n, n_heads, n_kv, max_seq);
+    // Shared key tiles where blocks of 128 queries cover three quarters of the CUs
+    // (256 CUs, us per layer, k_attn_prefill -> these, after 0 / 2048 / 6144 cached
+    // positions: 32 heads of 64, 768 positions 21.2 -> 13.5, 61 -> 34, 148 -> 92,
+    // 2048 77 -> 34, 190 -> 83, 416 -> 180; 32 heads of 128, 2048 185 -> 59, 467 -> 143,
+    // 1028 -> 314).
+    if (4 * n_heads * ((n + 127) / 128) >= 3 * num_cus) {
+        // Blocks of 64 queries: head_dim 128 (four partials of it do not fit a
+        // wave); of 64 while three blocks per CU take the whole chunk, or its
+        // causal triangle is most of the work (the last blocks are then short): us,
+        // 128 queries -> 64, 768 after 2048 48 -> 34, 1024 after 6144 132 -> 96, 2048 after 0
+        // 38 -> 34; past that 1555 after 2048 68 -> 76, 2048 after 2048 83 -> 92.
+        const int64_t b64 = (int64_t)n_heads * ((n + 63) / 64);
+        auto go = [&](auto kernel, int queries) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(n_heads * ((n + queries - 1) / queries))), dim3(256), 0, s, q, kc,
+                               vc, out, p0, n, n_heads, n_kv, max_seq);
+        };
+        if (hd == 128) go(k_attn_prefill_rows<128, 1>, 64);
+        else if (b64 <= 3 * (int64_t)num_cus || 4 * (int64_t)p0 < n) go(k_attn_prefill_rows<64, 1>, 64);
+        else go(k_attn_prefill_rows<64, 2>, 128);
         RQ_LAUNCH_CHECK();
         return RQ_OK;
     }
