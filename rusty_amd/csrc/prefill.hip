@@ -369,9 +369,8 @@ __global__ __launch_bounds__(NW * 64) void k_attn_prefill(const _Float16 *__rest
 // 16 matrix instructions per 64 keys at head_dim 64.  So the rest is kept off
 // every tile: the mask runs on a wave's last 32 keys only, and partials are
 // rescaled only when the maximum of one of their queries rose (the factor of the
-// others is exactly 1); a wave's two tiles are interleaved, as their chains of
-// matrix instructions, max, exchange and exponent are what it would wait for (one
-// after the other: 83 -> 92 us).
+// others is exactly 1); a wave's two tiles are written side by side, so that one's
+// matrix instructions can fill the other's wait for its max, exchange and exponent.
 template <int HD, int TPW>
 __global__ __launch_bounds__(256, HD == 64 && TPW == 1 ? 3 : 2) void k_attn_prefill_rows(
     const _Float16 *__restrict__ q, const _Float16 *__restrict__ kc, const _Float16 *__restrict__ vc,
